@@ -1,25 +1,20 @@
-// fft_kernels.hip -- LDS-staged mixed-radix (2, 3, 4, 5, 7) complex FFT along
-// one lattice axis, batched over every pencil of the 4 packed fields, with
-// the p^2 preconditioner fused into the last forward axis.
+// fft_kernels.hip -- LDS-staged mixed-radix (2, 3, 4, 5, 7, 8) complex FFT
+// along one or two lattice axes per pass, batched over every pencil of the 4
+// packed fields, with the p^2 preconditioner fused into the last forward
+// axis.
 //
 // This replaces the FFTW transforms of Gfix/FACG.c:77-95 (Landau, 4D) and
 // Gfix/CFACG.c:70-89 (Coulomb, 3D per time slice): forward transform,
 // multiply by psq = MAX / p^2 (Gfix/Landau.c:278-284), backward transform,
 // both unnormalised.
 //
-// A workgroup stages P pencils of length N in LDS (N*P <= 2048 complex),
-// runs a Stockham auto-sort radix-4/2/3 sequence on them, and writes them
-// back.  Pencils along x are contiguous rows; along y, z, t consecutive
+// A workgroup stages pencils in LDS, runs a Stockham auto-sort sequence of
+// radix stages on them, and writes them back.  Pencils along x are contiguous rows; along y, z, t consecutive
 // pencils are consecutive addresses, so loads and stores are coalesced in
 // both cases.  Twiddles come from a per-axis table computed on the host.
 #include "gfix_kernels.h"
 
 namespace gfix {
-
-template <typename T> __device__ __forceinline__ cx<T> tw_at(const double2 *tw, int idx, int sign) {
-  const double2 w = tw[idx];
-  return mk<T>((T)w.x, sign < 0 ? (T)w.y : (T)-w.y);
-}
 
 template <typename T, int R> __device__ __forceinline__ void dft_small(cx<T> (&v)[R], int sign) {
   if constexpr (R == 2) {
@@ -54,7 +49,7 @@ template <typename T, int R> __device__ __forceinline__ void dft_small(cx<T> (&v
       v[k + 4] = csub(e[k], w[k]);
     }
   } else if constexpr (R == 5 || R == 7) {
-    // plain O(R^2) DFT for the odd primes GLU's extents may contain
+    // the odd primes GLU's extents may contain
     constexpr double c5[5] = {1.0, 0.30901699437494745, -0.8090169943749475, -0.8090169943749475,
                               0.30901699437494745};
     constexpr double s5[5] = {0.0, 0.9510565162951535, 0.5877852522924731, -0.5877852522924731,
@@ -63,6 +58,33 @@ template <typename T, int R> __device__ __forceinline__ void dft_small(cx<T> (&v
                               -0.9009688679024191, -0.22252093395631434, 0.6234898018587336};
     constexpr double s7[7] = {0.0, 0.7818314824680298, 0.9749279121818236, 0.43388373911755823,
                               -0.43388373911755823, -0.9749279121818236, -0.7818314824680298};
+    if constexpr (sizeof(T) == 8) {
+      // the inputs q and R - q share their cosines and, up to sign, their
+      // sines: half the products and registers of the plain sums, which
+      // FP32 keeps (its rounding decides the FP32 phase's trajectory)
+      constexpr int H = (R - 1) / 2;
+      cx<T> a[H + 1], b[H + 1], y0 = v[0];
+#pragma unroll
+      for (int q = 1; q <= H; q++) {
+        a[q] = cadd(v[q], v[R - q]);
+        b[q] = cscale(csub(v[q], v[R - q]), (T)sign);
+        y0 = cadd(y0, a[q]);
+      }
+#pragma unroll
+      for (int m = 1; m <= H; m++) {
+        cx<T> A = v[0], B = mk<T>(T(0), T(0));
+#pragma unroll
+        for (int q = 1; q <= H; q++) {
+          const int k = (q * m) % R;
+          A = cadd(A, cscale(a[q], (T)(R == 5 ? c5[k] : c7[k])));
+          B = cadd(B, cscale(b[q], (T)(R == 5 ? s5[k] : s7[k])));
+        }
+        v[m] = mk<T>(A.re - B.im, A.im + B.re);  // A + i B
+        v[R - m] = mk<T>(A.re + B.im, A.im - B.re);
+      }
+      v[0] = y0;
+      return;
+    }
     cx<T> y[R];
 #pragma unroll
     for (int m = 0; m < R; m++) {
@@ -91,134 +113,208 @@ template <typename T, int R> __device__ __forceinline__ void dft_small(cx<T> (&v
 }
 
 constexpr int kFftThreads = 256;
-constexpr int kFftMaxItems = 4;
 
-// one Stockham stage of radix R on P pencils of length N held in LDS
+// ---------------------------------------------------------------------------
+// Any extents: one or two axes of a tile per pass, plans at run time
+// ---------------------------------------------------------------------------
+// The pass for extents without a compile-time kernel below: it transforms
+// the two axes of an x-y plane, the z and t axes of a column (forward z, t,
+// x p^2, backward t, z), or one axis, so that a lattice of any extents goes
+// through three passes over the fields like the common ones.  The tile sits
+// in LDS twice and every stage reads one copy and writes the other: one
+// barrier a stage, no values held across it, so a stage may have any number
+// of butterflies per thread.  Indices come from multipliers (the GPU has no
+// integer divide), and a stage's twiddle index q k N / (Ns R) is below N by
+// construction.  The arithmetic of a pencil is that of the compile-time
+// kernels: the same radix plan, twiddles and p^2 order.
+// On 20x28x10x36 in FP64 a Fourier acceleration took seven single-axis
+// passes of 30 us, bound by integer division; the three passes here take
+// 21 us each, bound by the issue of index and LDS instructions (FP32 takes
+// 17; a copy at 5.2 TB/s would take 5).
+struct AnyStage {
+  int R, Ns, nbf, tstep;
+  unsigned mNs;
+};
+struct AnyAxis {
+  int N, nst;
+  AnyStage st[8];
+  const double2 *tw;
+};
+// pencils of one axis in the tile: pencil j at (j % PJ) SJ + (j / PJ) PS,
+// its points SN apart
+struct AnyPencils {
+  int P, SN, SJ, PJ, PS;
+  unsigned mP, mPJ;
+};
+// what a tile is: m x-y planes (two axes), m neighbouring x-y sites' z-t
+// planes (two axes), m contiguous rows or m neighbouring pencils (one axis).
+// A template argument: a tile layout chosen at run time inside the kernel
+// left the compiler with a load address that one of the layouts never set.
+enum { ANY_PLANE = 0, ANY_COLUMN = 1, ANY_ROW = 2, ANY_AXIS = 3 };
+constexpr int any_axes(int lay) { return lay == ANY_PLANE || lay == ANY_COLUMN ? 2 : 1; }
+struct AnyPass {
+  AnyAxis ax[2];
+  AnyPencils pe[2];
+  int mode;
+  int m;            // planes, x-y sites or pencils per tile
+  int ld;           // LDS row length
+  int elems, pool;  // tile elements, LDS elements of one copy
+  unsigned mRow;    // division of an element index by the memory row
+  unsigned mZ;      // by the column's NZ
+  long long S, St;  // memory strides of the axes
+};
+
+inline unsigned any_mul(unsigned d) { return 0x80000000u / d + 1u; }
+// n / d for n d < 2^31, m = any_mul(d), d >= 1
+__device__ __forceinline__ unsigned any_div(unsigned n, unsigned m) { return __umulhi(2u * n, m); }
+
 template <typename T, int R>
-__device__ __forceinline__ void fft_stage(vec2<T> *lds, int ldP, int N, int P, int Ns, const double2 *tw,
-                                          int sign) {
-  const int nbf = N / R;
-  const int total = nbf * P;
-  const int tstep = N / (Ns * R);
-  cx<T> v[kFftMaxItems][R];
+__device__ __forceinline__ void any_stage(const vec2<T> *src, vec2<T> *dst, const AnyPencils &pe,
+                                          const AnyStage &sg, const vec2<T> *tw, int sign) {
+  const int total = sg.nbf * pe.P, Ns = sg.Ns;
+  for (int w = threadIdx.x; w < total; w += blockDim.x) {
+    const int b = (int)any_div((unsigned)w, pe.mP), j = w - b * pe.P;
+    const int g = pe.PJ == pe.P ? 0 : (int)any_div((unsigned)j, pe.mPJ);
+    const int jo = (j - g * pe.PJ) * pe.SJ + g * pe.PS;
+    const int h = (int)any_div((unsigned)b, sg.mNs), k = b - h * Ns;
+    cx<T> v[R];
 #pragma unroll
-  for (int it = 0; it < kFftMaxItems; it++) {
-    const int w = threadIdx.x + it * kFftThreads;
-    if (w < total) {
-      const int j = w % P, b = w / P, k = b % Ns;
+    for (int q = 0; q < R; q++) v[q] = ld<T>(src + (b + q * sg.nbf) * pe.SN + jo);
+    if (Ns > 1) {
+      const int kt = k * sg.tstep;
 #pragma unroll
-      for (int q = 0; q < R; q++) v[it][q] = ld<T>(lds + (b + q * nbf) * ldP + j);
-      if (Ns > 1) {
-#pragma unroll
-        for (int q = 1; q < R; q++) v[it][q] = cmul(v[it][q], tw_at<T>(tw, (q * k * tstep) % N, sign));
+      for (int q = 1; q < R; q++) {
+        cx<T> t = ld<T>(tw + q * kt);
+        if (sign > 0) t.im = -t.im;
+        v[q] = cmul(v[q], t);
       }
-      dft_small<T, R>(v[it], sign);
     }
-  }
-  __syncthreads();
+    dft_small<T, R>(v, sign);
+    const int out = h * Ns * R + k;
 #pragma unroll
-  for (int it = 0; it < kFftMaxItems; it++) {
-    const int w = threadIdx.x + it * kFftThreads;
-    if (w < total) {
-      const int j = w % P, b = w / P, k = b % Ns;
-      const int out = (b / Ns) * Ns * R + k;
-#pragma unroll
-      for (int q = 0; q < R; q++) st<T>(lds + (out + q * Ns) * ldP + j, v[it][q]);
-    }
+    for (int q = 0; q < R; q++) st<T>(dst + (out + q * Ns) * pe.SN + jo, v[q]);
   }
   __syncthreads();
 }
 
-template <typename T>
-__device__ __forceinline__ void fft_run(vec2<T> *lds, int ldP, const FftAxis &ax, int sign) {
-  int Ns = 1;
-  for (int s = 0; s < ax.nst; s++) {
-    const int R = ax.rad[s];
-    if (R == 4)
-      fft_stage<T, 4>(lds, ldP, ax.N, ax.P, Ns, ax.tw, sign);
-    else if (R == 2)
-      fft_stage<T, 2>(lds, ldP, ax.N, ax.P, Ns, ax.tw, sign);
-    else if (R == 3)
-      fft_stage<T, 3>(lds, ldP, ax.N, ax.P, Ns, ax.tw, sign);
-    else if (R == 5)
-      fft_stage<T, 5>(lds, ldP, ax.N, ax.P, Ns, ax.tw, sign);
-    else
-      fft_stage<T, 7>(lds, ldP, ax.N, ax.P, Ns, ax.tw, sign);
-    Ns *= R;
+// element e of a tile: its offset in memory and in LDS
+template <int LAY> __device__ __forceinline__ void any_place(const AnyPass &p, int e, long long &mem, int &lds) {
+  const int r = (int)any_div((unsigned)e, p.mRow);
+  if constexpr (LAY == ANY_COLUMN) {  // (j, z, t): e = j + m (z + NZ t)
+    const int t = (int)any_div((unsigned)r, p.mZ), NZ = p.ax[0].N;
+    mem = (e - r * p.m) + (long long)(r - t * NZ) * p.S + (long long)t * p.St;
+    lds = t * p.ld + (e - t * NZ * p.m);
+  } else if constexpr (LAY == ANY_AXIS) {  // (j, n): e = j + m n
+    mem = (e - r * p.m) + (long long)r * p.S;
+    lds = r * p.ld + (e - r * p.m);
+  } else {  // rows of N contiguous elements, one LDS column each
+    mem = e;
+    lds = (e - r * p.ax[0].N) * p.ld + r;
   }
 }
 
-// mode: 0 forward, 1 backward, 2 forward * psq * backward
-// blockIdx.z selects a batch slice of slice_len elements (Coulomb: one time
-// slice); slices with slice_done[z] set are skipped
-template <typename T>
-__global__ __launch_bounds__(kFftThreads) void k_fft_axis(vec2<T> *__restrict__ F, long long fstride, FftAxis ax,
-                                                         int mode, PsqInfo ps, const Ctrl *__restrict__ ctrl,
-                                                         long long slice_len, const int *__restrict__ slice_done,
-    const int *__restrict__ slice_map) {
+// mode: 0 forward, 1 backward, 2 forward, x p^2, backward.  blockIdx.y is
+// the field, blockIdx.z a batch slice (Coulomb: one time slice)
+template <typename T, int LAY, int POOL, int NTHR>
+__global__ __launch_bounds__(NTHR) void k_fft_any(vec2<T> *__restrict__ F, long long fstride, AnyPass p, PsqInfo ps,
+                                                 const Ctrl *__restrict__ ctrl, long long slice_len,
+                                                 const int *__restrict__ slice_done,
+                                                 const int *__restrict__ slice_map) {
+  constexpr int NAX = any_axes(LAY);
   if (ctrl && ctrl->done) return;
   // batch row blockIdx.z is time slice zs (the rows of running slices only)
   const int zs = slice_map ? slice_map[blockIdx.z] : (int)blockIdx.z;
   if (slice_done && slice_done[zs]) return;
-  extern __shared__ unsigned char fft_smem[];
-  vec2<T> *lds = reinterpret_cast<vec2<T> *>(fft_smem);
-  vec2<T> *base = F + (long long)blockIdx.y * fstride + (long long)zs * slice_len;
-  const long long p0 = (long long)blockIdx.x * ax.P;
-  const int ldP = ax.P + 1;
-  const int tot = ax.N * ax.P;
-  for (int idx = threadIdx.x; idx < tot; idx += kFftThreads) {
-    int n, j;
-    if (ax.S == 1) {
-      j = idx / ax.N;
-      n = idx % ax.N;
-    } else {
-      j = idx % ax.P;
-      n = idx / ax.P;
+  __shared__ vec2<T> pool[POOL];
+  int cur = 0, alt = p.pool;
+  const int tw0 = 2 * p.pool;  // the twiddles of axis 0, then of axis 1
+#pragma unroll
+  for (int x = 0; x < NAX; x++)
+    for (int k = threadIdx.x; k < p.ax[x].N; k += NTHR) {
+      const double2 w = p.ax[x].tw[k];
+      st<T>(pool + tw0 + x * p.ax[0].N + k, mk<T>((T)w.x, (T)w.y));
     }
-    const long long p = p0 + j;
-    if (p < ax.npencil) {
-      const long long gi = (p % ax.S) + (p / ax.S) * ax.S * ax.N + (long long)n * ax.S;
-      lds[n * ldP + j] = base[gi];
+  // neighbouring tiles share cache lines: each XCD gets a contiguous run
+  const unsigned nb = gridDim.x;
+  const unsigned tile = (nb & 7u) ? blockIdx.x : (blockIdx.x & 7u) * (nb >> 3) + (blockIdx.x >> 3);
+  long long first;  // first site of the tile
+  if constexpr (LAY == ANY_COLUMN) {
+    first = (long long)tile * p.m;
+  } else if constexpr (LAY == ANY_AXIS) {
+    const unsigned p0 = tile * (unsigned)p.m, q = p0 / (unsigned)p.S;
+    first = (long long)(p0 - q * (unsigned)p.S) + (long long)q * p.S * p.ax[0].N;
+  } else {
+    first = (long long)tile * p.elems;
+  }
+  vec2<T> *base = F + (long long)blockIdx.y * fstride + (long long)zs * slice_len + first;
+  // four loads in flight per thread before their LDS stores; past the end
+  // the last element is stored again
+  for (int e0 = threadIdx.x; e0 < p.elems; e0 += 4 * NTHR) {
+    vec2<T> v[4];
+    int lds[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      long long mem;
+      any_place<LAY>(p, min(e0 + k * NTHR, p.elems - 1), mem, lds[k]);
+      v[k] = base[mem];
     }
+#pragma unroll
+    for (int k = 0; k < 4; k++) pool[lds[k]] = v[k];
   }
   __syncthreads();
-  fft_run<T>(lds, ldP, ax, mode == 1 ? +1 : -1);
-  if (mode == 2) {
-    for (int idx = threadIdx.x; idx < tot; idx += kFftThreads) {
-      const int j = idx % ax.P, n = idx / ax.P;
-      const long long p = p0 + j;
-      if (p < ax.npencil) {
-        long long gi = (p % ax.S) + (p / ax.S) * ax.S * ax.N + (long long)n * ax.S;
-        // p^2 with the zero mode set to 1: Geometry/geometry.c:170-186
+  // the axes in order: forward 0, 1; backward 1, 0; mode 2 both in turn
+  const int steps = p.mode == 2 ? 2 * NAX : NAX;
+#pragma unroll 1
+  for (int i = 0; i < steps; i++) {
+    const bool back = p.mode == 1 || i >= NAX;
+    const int x = NAX == 1 ? 0 : (back ? (p.mode == 1 ? NAX : 2 * NAX) - 1 - i : i);
+    if (i == NAX) {
+      // p^2 with the zero mode set to 1 (Geometry/geometry.c:170-186), the
+      // cos of x, y, z, t added in that order
+      for (int e = threadIdx.x; e < p.elems; e += NTHR) {
+        long long mem;
+        int lds;
+        any_place<LAY>(p, e, mem, lds);
+        unsigned r = (unsigned)(first + mem);
         double kcos = 0.0;
         for (int mu = 0; mu < ps.D; mu++) {
-          const int xm = (int)(gi % ps.L[mu]);
-          gi /= ps.L[mu];
-          kcos += ps.cosv[ps.off[mu] + xm];
+          const unsigned q = __umulhi(r, ps.dm[mu]) >> ps.ds[mu];
+          kcos += ps.cosv[ps.off[mu] + (int)(r - q * (unsigned)ps.L[mu])];
+          r = q;
         }
         const double p2 = (kcos == (double)ps.D) ? 1.0 : 2.0 * ((double)ps.D - kcos);
         const T f = (T)(ps.max / p2);
-        cx<T> z = ld<T>(lds + n * ldP + j);
-        st<T>(lds + n * ldP + j, mk<T>(z.re * f, z.im * f));
+        const cx<T> z = ld<T>(pool + cur + lds);
+        st<T>(pool + cur + lds, mk<T>(z.re * f, z.im * f));
       }
+      __syncthreads();
     }
-    __syncthreads();
-    fft_run<T>(lds, ldP, ax, +1);
+    const AnyAxis &ax = p.ax[x];
+    const AnyPencils pe = p.pe[x];
+    const vec2<T> *tw = pool + tw0 + x * p.ax[0].N;
+    for (int s = 0; s < ax.nst; s++) {
+      const AnyStage sg = ax.st[s];
+      const vec2<T> *src = pool + cur;
+      vec2<T> *dst = pool + alt;
+      const int sign = back ? +1 : -1;
+      switch (sg.R) {
+        case 2: any_stage<T, 2>(src, dst, pe, sg, tw, sign); break;
+        case 3: any_stage<T, 3>(src, dst, pe, sg, tw, sign); break;
+        case 4: any_stage<T, 4>(src, dst, pe, sg, tw, sign); break;
+        case 5: any_stage<T, 5>(src, dst, pe, sg, tw, sign); break;
+        case 7: any_stage<T, 7>(src, dst, pe, sg, tw, sign); break;
+        default: any_stage<T, 8>(src, dst, pe, sg, tw, sign); break;
+      }
+      const int t = cur;
+      cur = alt;
+      alt = t;
+    }
   }
-  for (int idx = threadIdx.x; idx < tot; idx += kFftThreads) {
-    int n, j;
-    if (ax.S == 1) {
-      j = idx / ax.N;
-      n = idx % ax.N;
-    } else {
-      j = idx % ax.P;
-      n = idx / ax.P;
-    }
-    const long long p = p0 + j;
-    if (p < ax.npencil) {
-      const long long gi = (p % ax.S) + (p / ax.S) * ax.S * ax.N + (long long)n * ax.S;
-      base[gi] = lds[n * ldP + j];
-    }
+  for (int e = threadIdx.x; e < p.elems; e += NTHR) {
+    long long mem;
+    int lds;
+    any_place<LAY>(p, e, mem, lds);
+    base[mem] = pool[cur + lds];
   }
 }
 
@@ -349,6 +445,159 @@ __global__ __launch_bounds__(kFftThreads) void k_fft_xy(vec2<T> *__restrict__ F,
   for (int e = threadIdx.x; e < NT; e += kFftThreads) base[e] = lds[(e % NX) * LD + e / NX];
 }
 
+// ---- launches of the run-time pass
+// extents with compile-time kernels keep their radix order (8 first)
+static bool fast_extent(int N) {
+  for (int n : {4, 6, 8, 12, 16, 24, 32, 48, 64, 96})
+    if (n == N) return true;
+  return false;
+}
+static AnyAxis any_axis_plan(const FftAxis &ax) {
+  AnyAxis a{};
+  a.N = ax.N;
+  a.tw = ax.tw;
+  const RadPlan fast = make_plan(ax.N);
+  const bool f = fast_extent(ax.N);
+  a.nst = f ? fast.n : ax.nst;
+  int Ns = 1;
+  for (int s = 0; s < a.nst; s++) {
+    const int R = f ? fast.r[s] : ax.rad[s];
+    a.st[s] = AnyStage{(unsigned short)R, (unsigned short)Ns, (unsigned short)(ax.N / R),
+                       (unsigned short)(ax.N / (Ns * R)), any_mul((unsigned)Ns)};
+    Ns *= R;
+  }
+  return a;
+}
+static AnyPencils any_pencils(int P, int SN, int SJ, int PJ, int PS) {
+  return AnyPencils{P, SN, SJ, PJ, PS, any_mul((unsigned)P), any_mul((unsigned)PJ)};
+}
+// LDS of a workgroup in complex numbers: 40, 80 and 160 KB in FP64 (4, 2
+// and 1 workgroups per CU), half of that in FP32
+constexpr int kAnyPool[3] = {2560, 5120, 10000};
+
+// the largest divisor m of n whose tile (need(m) LDS numbers) fits `pool`
+// and leaves at least `least` tiles; 0 if not even m = 1 fits
+template <typename Need> static int any_split(long long n, int pool, long long least, Need need) {
+  int best = 0;
+  for (int m = 1; m <= n && m <= 256; m++) {
+    if (n % m) continue;
+    if (need(m) > pool) break;
+    if (m > 1 && n / m < least) break;
+    best = m;
+  }
+  return best;
+}
+
+template <typename T, int LAY>
+static void launch_any(void *F, long long fstride, int nfield, const AnyPass &p, unsigned tiles, const PsqInfo &ps,
+                       const Ctrl *ctrl, hipStream_t s, int nslice, long long slice_len, const int *slice_done,
+                       const int *slice_map) {
+  const int need = 2 * p.pool + p.ax[0].N + (any_axes(LAY) > 1 ? p.ax[1].N : 0);
+  const dim3 grid(tiles, nfield, nslice);
+  if (need <= kAnyPool[0])
+    hipLaunchKernelGGL((k_fft_any<T, LAY, kAnyPool[0], 256>), grid, dim3(256), 0, s, (vec2<T> *)F, fstride, p, ps, ctrl,
+                       slice_len, slice_done, slice_map);
+  else if (need <= kAnyPool[1])
+    hipLaunchKernelGGL((k_fft_any<T, LAY, kAnyPool[1], 512>), grid, dim3(512), 0, s, (vec2<T> *)F, fstride, p, ps, ctrl,
+                       slice_len, slice_done, slice_map);
+  else
+    hipLaunchKernelGGL((k_fft_any<T, LAY, kAnyPool[2], 512>), grid, dim3(512), 0, s, (vec2<T> *)F, fstride, p, ps, ctrl,
+                       slice_len, slice_done, slice_map);
+}
+
+// Tiles a pass is split into at least.  Per pass on 28x36x42x32 FP64: 85 us
+// with 256 or 512 tiles, 90 with 1024, 84 with 2048; on 20x28x10x36 21.3, 23
+// and 25 us with 512, 1024 and 2048, and 12x12x12x24 11.4 us with up to 512,
+// 13 above
+constexpr long long kAnyTiles = 512;
+
+// x-y planes of any extents (false when a plane does not fit the LDS)
+template <typename T>
+static bool any_plane(void *F, long long fstride, int nfield, const FftAxis &ax, const FftAxis &ay, int mode,
+                      const Ctrl *ctrl, hipStream_t s, long long nplane, int nslice, long long slice_len,
+                      const int *slice_done, const int *slice_map) {
+  const int NX = ax.N, NY = ay.N;
+  auto need = [&](int m) { return 2 * NX * ((m * NY) | 1) + NX + NY; };
+  if ((long long)NX * NY > kAnyPool[2] || need(1) > kAnyPool[2]) return false;
+  int m = any_split(nplane, kAnyPool[0], kAnyTiles / ((long long)nfield * nslice) + 1, need);
+  if (!m) m = 1;
+  AnyPass p{};
+  p.mode = mode;
+  p.m = m;
+  p.ld = (m * NY) | 1;
+  p.elems = m * NX * NY;
+  p.pool = NX * p.ld;
+  p.mRow = any_mul((unsigned)NX);
+  p.S = 1;
+  p.ax[0] = any_axis_plan(ax);
+  p.ax[1] = any_axis_plan(ay);
+  p.pe[0] = any_pencils(m * NY, p.ld, 1, m * NY, 0);   // x pencil (plane, y)
+  p.pe[1] = any_pencils(m * NX, 1, p.ld, NX, NY);      // y pencil (plane, x)
+  launch_any<T, ANY_PLANE>(F, fstride, nfield, p, (unsigned)(nplane / m), PsqInfo{}, ctrl, s, nslice, slice_len, slice_done,
+                slice_map);
+  return true;
+}
+
+// z-t columns of any extents, m neighbouring x-y sites per tile.  The
+// smallest LDS pool that holds a column: longer runs in a larger pool were
+// no faster (36x36x36x40 FP64: 127 us per pass with runs of 16 B, 128 with
+// 64), the columns of one XCD share the lines in its L2
+template <typename T>
+static bool any_column(void *F, long long V, int nfield, const FftAxis &ax, const FftAxis &ay, const FftAxis &az,
+                       const FftAxis &at, const PsqInfo &ps, const Ctrl *ctrl, hipStream_t s, bool launch) {
+  const int NZ = az.N, NT = at.N;
+  const long long nxy = (long long)ax.N * ay.N;
+  auto need = [&](int m) { return 2 * NT * ((m * NZ) | 1) + NZ + NT; };
+  if ((long long)NZ * NT > kAnyPool[2] || need(1) > kAnyPool[2]) return false;
+  if (!launch) return true;
+  int m = 0;
+  for (int k = 0; k < 3 && !m; k++) m = any_split(nxy, kAnyPool[k], kAnyTiles / nfield, need);
+  AnyPass p{};
+  p.mode = 2;
+  p.m = m;
+  p.ld = (m * NZ) | 1;
+  p.elems = m * NZ * NT;
+  p.pool = NT * p.ld;
+  p.mRow = any_mul((unsigned)m);
+  p.mZ = any_mul((unsigned)NZ);
+  p.S = nxy;
+  p.St = nxy * NZ;
+  p.ax[0] = any_axis_plan(az);
+  p.ax[1] = any_axis_plan(at);
+  p.pe[0] = any_pencils(m * NT, m, 1, m, p.ld);       // z pencil (t, j)
+  p.pe[1] = any_pencils(m * NZ, p.ld, 1, m * NZ, 0);  // t pencil (z, j)
+  launch_any<T, ANY_COLUMN>(F, V, nfield, p, (unsigned)(nxy / m), ps, ctrl, s, 1, 0, nullptr, nullptr);
+  return true;
+}
+
+// one axis of any extent: m pencils per tile, neighbours in memory (m
+// divides the stride, so a tile never straddles two pencil rows)
+template <typename T>
+static void any_single(void *F, long long fstride, int nfield, const FftAxis &ax, int mode, const PsqInfo &ps,
+                       const Ctrl *ctrl, hipStream_t s, int nslice, long long slice_len, const int *slice_done,
+                       const int *slice_map) {
+  const int N = ax.N;
+  auto need = [&](int m) { return 2 * N * (m | 1) + N; };
+  const long long n = ax.S == 1 ? ax.npencil : ax.S;
+  int m = any_split(n, kAnyPool[0], 1, need);
+  if (!m) m = 1;  // N up to 2048: 3 N numbers fit the largest pool
+  AnyPass p{};
+  p.mode = mode;
+  p.m = m;
+  p.ld = m | 1;
+  p.elems = m * N;
+  p.pool = N * p.ld;
+  p.mRow = any_mul((unsigned)(ax.S == 1 ? N : m));
+  p.S = ax.S;
+  p.ax[0] = any_axis_plan(ax);
+  p.pe[0] = any_pencils(m, p.ld, 1, m, 0);
+  const unsigned tiles = (unsigned)(ax.npencil / m);
+  if (ax.S == 1)
+    launch_any<T, ANY_ROW>(F, fstride, nfield, p, tiles, ps, ctrl, s, nslice, slice_len, slice_done, slice_map);
+  else
+    launch_any<T, ANY_AXIS>(F, fstride, nfield, p, tiles, ps, ctrl, s, nslice, slice_len, slice_done, slice_map);
+}
+
 template <typename T, int N>
 static bool try_xy(void *F, long long fstride, int nfield, const FftAxis &ax, const FftAxis &ay, int mode,
                    const Ctrl *ctrl, hipStream_t s, long long nplane, int nslice, long long slice_len,
@@ -376,7 +625,8 @@ bool launch_fft_xy(void *F, long long fstride, int nfield, const FftAxis &ax, co
          try_xy<T, 16>(F, fstride, nfield, ax, ay, mode, ctrl, s, nplane, nslice, slice_len, slice_done, slice_map) ||
          try_xy<T, 24>(F, fstride, nfield, ax, ay, mode, ctrl, s, nplane, nslice, slice_len, slice_done, slice_map) ||
          try_xy<T, 32>(F, fstride, nfield, ax, ay, mode, ctrl, s, nplane, nslice, slice_len, slice_done, slice_map) ||
-         try_xy<T, 48>(F, fstride, nfield, ax, ay, mode, ctrl, s, nplane, nslice, slice_len, slice_done, slice_map);
+         try_xy<T, 48>(F, fstride, nfield, ax, ay, mode, ctrl, s, nplane, nslice, slice_len, slice_done, slice_map) ||
+         any_plane<T>(F, fstride, nfield, ax, ay, mode, ctrl, s, nplane, nslice, slice_len, slice_done, slice_map);
 }
 template bool launch_fft_xy<double>(void *, long long, int, const FftAxis &, const FftAxis &, int, const Ctrl *,
                                     hipStream_t, long long, int, long long, const int *, const int *);
@@ -513,7 +763,8 @@ bool launch_fft_zt(void *F, long long V, int nfield, const FftAxis &ax, const Ff
          try_zt<T, 16, 16>(F, V, nfield, ax, ay, az, at, ps, ctrl, s, launch, v) ||
          try_zt<T, 16, 32>(F, V, nfield, ax, ay, az, at, ps, ctrl, s, launch, v) ||
          try_zt<T, 24, 48>(F, V, nfield, ax, ay, az, at, ps, ctrl, s, launch, v) ||
-         try_zt<T, 32, 64>(F, V, nfield, ax, ay, az, at, ps, ctrl, s, launch, v);
+         try_zt<T, 32, 64>(F, V, nfield, ax, ay, az, at, ps, ctrl, s, launch, v) ||
+         (v == 0 && any_column<T>(F, V, nfield, ax, ay, az, at, ps, ctrl, s, launch));
 }
 template bool launch_fft_zt<double>(void *, long long, int, const FftAxis &, const FftAxis &, const FftAxis &,
                                     const FftAxis &, const PsqInfo &, const Ctrl *, hipStream_t, bool, int);
@@ -639,10 +890,7 @@ void launch_fft_axis(void *F, long long fstride, int nfield, const FftAxis &ax, 
       try_fast<T, 64>(F, fstride, nfield, ax, mode, ps, ctrl, s, nslice, slice_len, slice_done, slice_map) ||
       try_fast<T, 96>(F, fstride, nfield, ax, mode, ps, ctrl, s, nslice, slice_len, slice_done, slice_map))
     return;
-  const unsigned nb = (unsigned)((ax.npencil + ax.P - 1) / ax.P);
-  const size_t sm = (size_t)ax.N * (ax.P + 1) * sizeof(vec2<T>);
-  hipLaunchKernelGGL(k_fft_axis<T>, dim3(nb, nfield, nslice), dim3(kFftThreads), sm, s, (vec2<T> *)F, fstride, ax,
-                     mode, ps, ctrl, slice_len, slice_done, slice_map);
+  any_single<T>(F, fstride, nfield, ax, mode, ps, ctrl, s, nslice, slice_len, slice_done, slice_map);
 }
 template void launch_fft_axis<double>(void *, long long, int, const FftAxis &, int, const PsqInfo &, const Ctrl *,
                                       hipStream_t, int, long long, const int *, const int *);

@@ -63,12 +63,6 @@ int factor_radices(int N, int *rad) {
   return N == 1 ? n : -1;
 }
 
-size_t pow2_floor(size_t x) {
-  size_t p = 1;
-  while (p * 2 <= x) p *= 2;
-  return p;
-}
-
 }  // namespace
 
 size_t gfix_footprint(const size_t dims[4], int gftype, int precision) {
@@ -103,6 +97,8 @@ void fft_plan(glu_gfix_ctx *c, double2 *const tw[4], double *cosv) {
     const int N = c->g.L[mu];
     c->ps.off[mu] = off;
     c->ps.L[mu] = N;
+    c->ps.dm[mu] = c->g.dm[mu];
+    c->ps.ds[mu] = c->g.ds[mu];
     const double twd = 6.283185307179586 / (double)N;
     for (int n = 0; n < N; n++) cosv[off + n] = cos(n * twd);
     off += N;
@@ -112,7 +108,6 @@ void fft_plan(glu_gfix_ctx *c, double2 *const tw[4], double *cosv) {
     ax.nst = factor_radices(N, ax.rad);
     ax.S = c->g.S[mu];
     ax.npencil = (D == 4 ? V : c->g.Lcu) / N;  // per transform (Coulomb: per slice)
-    ax.P = (int)std::min<size_t>(512, pow2_floor(2048 / (size_t)N));
     for (int k = 0; k < N; k++) {
       const double a = 6.283185307179586 * (double)k / (double)N;
       tw[mu][k] = make_double2(cos(a), -sin(a));

@@ -12,7 +12,6 @@ namespace gfix {
 // one FFT axis pass: pencils of length N at stride S
 struct FftAxis {
   int N;
-  int P;        // pencils per workgroup
   long long S;  // element stride along the axis
   long long npencil;
   int nst;
@@ -26,6 +25,8 @@ struct PsqInfo {
   int D;             // 4 Landau, 3 Coulomb
   int L[4];
   int off[4];        // offsets of each axis' cos table in cosv
+  unsigned dm[4];    // multipliers and shifts for division by L (as Geo's)
+  int ds[4];
   const double *cosv;
   double max;        // MAX_LANDAU = 4 ND / V or MAX_COULOMB = 4 (ND-1) / Lcu
 };
