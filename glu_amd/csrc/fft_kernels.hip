@@ -170,7 +170,7 @@ __device__ __forceinline__ unsigned any_div(unsigned n, unsigned m) { return __u
 
 template <typename T, int R>
 __device__ __forceinline__ void any_stage(const vec2<T> *src, vec2<T> *dst, const AnyPencils &pe,
-                                          const AnyStage &sg, const vec2<T> *tw, int sign) {
+                                          const AnyStage &sg, const vec2<T> *tw, const int sign) {
   const int total = sg.nbf * pe.P, Ns = sg.Ns;
   for (int w = threadIdx.x; w < total; w += blockDim.x) {
     const int b = (int)any_div((unsigned)w, pe.mP), j = w - b * pe.P;
@@ -297,13 +297,24 @@ __global__ __launch_bounds__(NTHR) void k_fft_any(vec2<T> *__restrict__ F, long 
       const vec2<T> *src = pool + cur;
       vec2<T> *dst = pool + alt;
       const int sign = back ? +1 : -1;
-      switch (sg.R) {
-        case 2: any_stage<T, 2>(src, dst, pe, sg, tw, sign); break;
-        case 3: any_stage<T, 3>(src, dst, pe, sg, tw, sign); break;
-        case 4: any_stage<T, 4>(src, dst, pe, sg, tw, sign); break;
-        case 5: any_stage<T, 5>(src, dst, pe, sg, tw, sign); break;
-        case 7: any_stage<T, 7>(src, dst, pe, sg, tw, sign); break;
-        default: any_stage<T, 8>(src, dst, pe, sg, tw, sign); break;
+      // In FP32 the compiler fuses the products of the radix-5 and radix-7
+      // sums by whether it knows the sign; the axis p^2 is applied on is
+      // transformed back with a known one, as it always has been, so that an
+      // FP32 trajectory keeps its rounding
+      if (sizeof(T) == 4 && i == NAX && (sg.R == 5 || sg.R == 7)) {
+        if (sg.R == 5)
+          any_stage<T, 5>(src, dst, pe, sg, tw, +1);
+        else
+          any_stage<T, 7>(src, dst, pe, sg, tw, +1);
+      } else {
+        switch (sg.R) {
+          case 2: any_stage<T, 2>(src, dst, pe, sg, tw, sign); break;
+          case 3: any_stage<T, 3>(src, dst, pe, sg, tw, sign); break;
+          case 4: any_stage<T, 4>(src, dst, pe, sg, tw, sign); break;
+          case 5: any_stage<T, 5>(src, dst, pe, sg, tw, sign); break;
+          case 7: any_stage<T, 7>(src, dst, pe, sg, tw, sign); break;
+          default: any_stage<T, 8>(src, dst, pe, sg, tw, sign); break;
+        }
       }
       const int t = cur;
       cur = alt;
@@ -452,6 +463,12 @@ static bool fast_extent(int N) {
     if (n == N) return true;
   return false;
 }
+// axes of 48 and 96 points stay with their compile-time passes in FP32: the
+// three-stage kernels round some products differently, and an FP32
+// trajectory follows the rounding
+template <typename T> static bool any_keeps_rounding(const FftAxis &ax) {
+  return sizeof(T) == 8 || (ax.N != 48 && ax.N != 96);
+}
 static AnyAxis any_axis_plan(const FftAxis &ax) {
   AnyAxis a{};
   a.N = ax.N;
@@ -518,6 +535,7 @@ static bool any_plane(void *F, long long fstride, int nfield, const FftAxis &ax,
                       const int *slice_done, const int *slice_map) {
   const int NX = ax.N, NY = ay.N;
   auto need = [&](int m) { return 2 * NX * ((m * NY) | 1) + NX + NY; };
+  if (!any_keeps_rounding<T>(ax) || !any_keeps_rounding<T>(ay)) return false;
   if ((long long)NX * NY > kAnyPool[2] || need(1) > kAnyPool[2]) return false;
   int m = any_split(nplane, kAnyPool[0], kAnyTiles / ((long long)nfield * nslice) + 1, need);
   if (!m) m = 1;
@@ -548,6 +566,7 @@ static bool any_column(void *F, long long V, int nfield, const FftAxis &ax, cons
   const int NZ = az.N, NT = at.N;
   const long long nxy = (long long)ax.N * ay.N;
   auto need = [&](int m) { return 2 * NT * ((m * NZ) | 1) + NZ + NT; };
+  if (!any_keeps_rounding<T>(az) || !any_keeps_rounding<T>(at)) return false;
   if ((long long)NZ * NT > kAnyPool[2] || need(1) > kAnyPool[2]) return false;
   if (!launch) return true;
   int m = 0;
