@@ -161,13 +161,6 @@ extern "C" int glu_gfix_create(glu_gfix_ctx **out, const size_t dims[4], int gft
   c->g.Lcu = c->g.S[3];
   geo_set_div(c->g);
   c->g.xcd = 0;
-  // untuned line search: tile 5 where the lattice takes it.  The tile
-  // fixes the summation order of the probes, and late in a solve the
-  // trajectory follows rounding: at 24^3x48 the autotuner's 32^3x64 pick
-  // (tile 2, 7% faster per FP64 iteration) ends one gauge copy on another
-  // Gribov copy than the CPU reference does in both of its orders
-  c->ls_tile = ls_tile_fits(c->g, 5) ? 5 : 0;
-  if (const char *e = getenv("GLU_GFIX_LS_TILE")) c->ls_tile = ls_tile_fits(c->g, atoi(e)) ? atoi(e) : 0;
   if (const char *e = getenv("GLU_GFIX_XCD")) {
     c->ord_eg = c->ord_ls = std::min(std::max(atoi(e), 0), 2);
     c->ord_cl = c->ord_eg ? 1 : 0;
@@ -555,7 +548,7 @@ template <typename T> static void enq_sd_start(glu_gfix_ctx *c, const Bufs &b) {
   launch_deriv<T>(b.U, b.F, c->part, geo_order(c, c->ord_eg), c->ctrl, s);
   launch_fin_theta(c->part, c->nblk, c->ctrl, landau_norm(c), s);
   enq_fa<T>(c, b.F, c->ctrl, nullptr);
-  launch_line_search<T>(b.U, b.F, c->part, geo_order(c, c->ord_ls), c->ctrl, 1, s, c->ls_tile);
+  launch_line_search<T>(b.U, b.F, c->part, geo_order(c, c->ord_ls), c->ctrl, 1, s);
   launch_fin_ls(c->part, c->nblk, c->ctrl, c->trace, 1, 0.15, 0.30, s);
   launch_copy<T>(b.F, b.sn, c->g.V, c->ctrl, s);
   launch_pr_sums<T>(b.F, b.F, c->part, c->g.V, c->ctrl, s);
@@ -579,7 +572,7 @@ template <typename T> static void enq_cg_iter(glu_gfix_ctx *c, const Bufs &b) {
   launch_fin_pr(c->part, c->nblk, c->ctrl, s);
   GFIX_PROF(c, pk<T>(PK_CGUPD), launch_cg_update<T>(b.F, b.sn, c->g.V, c->ctrl, s));
   GFIX_PROF(c, pk<T>(PK_LSEARCH),
-            launch_line_search<T>(b.U, b.sn, c->part, geo_order(c, c->ord_ls), c->ctrl, 0, s, c->ls_tile));
+            launch_line_search<T>(b.U, b.sn, c->part, geo_order(c, c->ord_ls), c->ctrl, 0, s));
   launch_fin_ls(c->part, c->nblk, c->ctrl, c->trace, 0, 0.15, 0.30, s);
   enq_update_deriv<T>(c);
   launch_fin_iter(c->part, c->nblk, c->ctrl, c->trace, landau_norm(c), s);
@@ -1140,7 +1133,7 @@ extern "C" int glu_gfix_stage_line_search(glu_gfix_ctx *c, const double *fields,
   if (c->gftype != GLU_GFIX_LANDAU) return gfix_fail(-1, "stage entry points are Landau-only");
   if (int rc = ctrl_live(c, 0.0, 1.0)) return rc;
   if (int rc = fields_in(c, fields, c->sn)) return rc;
-  launch_line_search<double>(c->U64, c->sn, c->part, c->g, c->ctrl, 1, c->stream, c->ls_tile);
+  launch_line_search<double>(c->U64, c->sn, c->part, c->g, c->ctrl, 1, c->stream);
   launch_fin_ls(c->part, c->nblk, c->ctrl, nullptr, 1, 0.15, 0.30, c->stream);
   if (int rc = read_ctrl(c)) return rc;
   for (int k = 0; k < 3; k++) probes[k] = c->hctrl->probe[k];

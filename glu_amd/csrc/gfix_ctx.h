@@ -81,9 +81,6 @@ struct glu_gfix_ctx {
   // workgroup order (Geo::xcd) of the derivative / fused update and of the
   // line search; set by the autotuner
   int ord_eg = 1, ord_ls = 1;
-  // line search on 256-site tiles (kLsTileShape[ls_tile - 1]; 0: one site
-  // per thread); set at creation, then by the autotuner
-  int ls_tile = 0;
   int ord_cl = 1;  // Coulomb slice stencils: XCD-contiguous (1) or plain (0)
   int use_graph = 0;  // replay iteration batches from captured HIP graphs
   // iterations enqueued between host checks; the iterations enqueued past

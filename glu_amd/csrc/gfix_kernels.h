@@ -64,17 +64,9 @@ template <typename T>
 void launch_cg_update(const void *F, void *sn, long long V, const Ctrl *ctrl, hipStream_t s);
 template <typename T>
 void launch_copy(const void *F, void *a, long long V, const Ctrl *ctrl, hipStream_t s);
-// the line search on 256-site tiles: variant k (1..kLsTiles) has the tile
-// kLsTileShape[k - 1] = (TX, TY, TZ, TT), the link columns held in
-// registers for both probes (k <= 4) or loaded per probe (k > 4); 0, or a
-// shape that does not divide the lattice, runs the one-site-per-thread kernel
-constexpr int kLsTiles = 8;
-constexpr int kLsTileShape[kLsTiles][4] = {{8, 4, 4, 2}, {4, 4, 4, 4}, {8, 8, 2, 2}, {16, 4, 2, 2},
-                                           {8, 4, 4, 2}, {4, 4, 4, 4}, {8, 8, 2, 2}, {16, 4, 2, 2}};
-bool ls_tile_fits(const Geo &g, int tile);
 template <typename T>
 void launch_line_search(const void *U, const void *F, double *part, const Geo &g, const Ctrl *ctrl, int force,
-                        hipStream_t s, int tile = 0);
+                        hipStream_t s);
 template <typename T>
 void launch_egauge(void *U, const void *F, void *G, const Geo &g, const Ctrl *ctrl, int fixed, hipStream_t s);
 template <typename T>

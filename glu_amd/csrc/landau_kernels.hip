@@ -99,14 +99,20 @@ __device__ __forceinline__ su3<T> gauge_at(const vec2<T> *__restrict__ F, long l
 // functional, so they are computed in FP64 whatever the storage type: in
 // FP32 the rounding of the reunitarised probe matrices biases the O(12 V)
 // sums by more than the differences the parabola fit needs.
+//
+// Bound by FP64 issue (about 2500 instructions a site).  Both probes are
+// taken in one pass: the links and the neighbours' fields are loaded and
+// converted once, and no third column of a link or a neighbour's matrix is
+// formed (retrace_cols).  In FP64 the two matrices of a site share their
+// inner products (ProbeSite); the FP32 phase builds each by Gram-Schmidt and
+// sums over 8 x 4 x 4 x 2 tiles, because its trajectory follows the rounding
+// of the step.  It runs at 2 waves per SIMD (218 VGPRs, 184 in FP32): the
+// two probes' chains fill the issue slots, where one probe at a time at 3
+// waves took 253 us and capped at 4 waves, spilling, 795.  32^3x64: 242 us
+// in FP64 (388 with the matrices shared through LDS on tiles, 306 with one
+// probe at a time and three-column traces), 238 from FP32 links (281 on LDS
+// tiles); the bytes alone would take 180 and 90.
 // ---------------------------------------------------------------------------
-template <typename T>
-__device__ __forceinline__ su3<double> promote(const su3<T> &m) {
-  su3<double> d;
-#pragma unroll
-  for (int k = 0; k < 9; k++) d.e[k] = mk<double>((double)m.e[k].re, (double)m.e[k].im);
-  return d;
-}
 template <typename T>
 __device__ __forceinline__ su3<double> gauge_at64(const vec2<T> *__restrict__ F, long long V, long long i,
                                                   double alpha) {
@@ -117,8 +123,95 @@ __device__ __forceinline__ su3<double> gauge_at64(const vec2<T> *__restrict__ F,
   return gauge_matrix<double>(f(i), f(V + i), f(2 * V + i), f(3 * V + i), alpha);
 }
 
+// the four packed field values at a site, in FP64
+template <typename T>
+__device__ __forceinline__ void field_at(const vec2<T> *__restrict__ F, long long V, long long i, cx<double> (&f)[4]) {
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const cx<T> z = ld<T>(F + k * V + i);
+    f[k] = mk<double>((double)z.re, (double)z.im);
+  }
+}
+// columns 0 and 1 of the two probe matrices of one site
+__device__ __forceinline__ void probe_cols(const cx<double> (&f)[4], cx<double> (&c)[2][6], double) {
+  ProbeSite s;
+  s.set(f[0], f[1], f[2], f[3]);
+  s.cols(0.15, c[0]);
+  s.cols(0.30, c[1]);
+}
+__device__ __forceinline__ void probe_cols(const cx<double> (&f)[4], cx<double> (&c)[2][6], float) {
+#pragma unroll
+  for (int pr = 0; pr < 2; pr++) {
+    const su3<double> m = gauge_cols01<double>(f[0], f[1], f[2], f[3], pr == 0 ? 0.15 : 0.30);
+    c[pr][0] = m.e[0], c[pr][1] = m.e[3], c[pr][2] = m.e[6];
+    c[pr][3] = m.e[1], c[pr][4] = m.e[4], c[pr][5] = m.e[7];
+  }
+}
+// site of this thread: in FP32 a workgroup owns an 8 x 4 x 4 x 2 tile
+__device__ __forceinline__ long long probe_site(const Geo &g, unsigned lb, double) {
+  return (long long)lb * blockDim.x + threadIdx.x;
+}
+__device__ __forceinline__ long long probe_site(const Geo &g, unsigned lb, float) {
+  const unsigned nx = (unsigned)g.L[0] / 8, ny = (unsigned)g.L[1] / 4, nz = (unsigned)g.L[2] / 4;
+  const unsigned t = threadIdx.x, by = lb / nx, bz = by / ny, bt = bz / nz;
+  const long long x = (lb - by * nx) * 8 + (t & 7u), y = (by - bz * ny) * 4 + (t >> 3 & 3u);
+  const long long z = (bz - bt * nz) * 4 + (t >> 5 & 3u), tt = bt * 2 + (t >> 7);
+  return x + g.S[1] * y + g.S[2] * z + g.S[3] * tt;
+}
+
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_line_search(const vec2<T> *__restrict__ U, const vec2<T> *__restrict__ F,
+                                                       double *__restrict__ part, Geo g,
+                                                       const Ctrl *__restrict__ ctrl, int force) {
+  if (ctrl->done) return;
+  if (!force && !(ctrl->theta > ctrl->cg_tol)) return;
+  const long long V = g.V;
+  const unsigned lb = logical_block(g);
+  const long long i = probe_site(g, lb, T(0));
+  double v[3] = {0.0, 0.0, 0.0};
+  if (i < V) {
+    int x[4];
+    coords(g, i, x);
+    cx<double> A[2][6];
+    {
+      cx<double> f[4];
+      field_at<T>(F, V, i, f);
+      probe_cols(f, A, T(0));
+    }
+#pragma unroll 1
+    for (int mu = 0; mu < kND; mu++) {
+      cx<double> u[6], f[4], B[2][6];
+#pragma unroll
+      for (int k = 0; k < 6; k++) {
+        const cx<T> w = ld<T>(U + ((long long)mu * 6 + k) * V + i);
+        u[k] = mk<double>((double)w.re, (double)w.im);
+      }
+      field_at<T>(F, V, nb_fwd(g, i, x, mu), f);
+      // Re tr u, its third diagonal entry conj(U00 U11 - U10 U01)
+      v[0] += u[0].re + u[4].re + (u[0].re * u[4].re - u[0].im * u[4].im) -
+              (u[1].re * u[3].re - u[1].im * u[3].im);
+      probe_cols(f, B, T(0));
+#pragma unroll
+      for (int pr = 0; pr < 2; pr++) {
+        const cx<double> *a = A[pr];
+        const cx<double> a2[3] = {third(a[1], a[2], a[4], a[5]), third(a[2], a[0], a[5], a[3]),
+                                  third(a[0], a[1], a[3], a[4])};
+        v[1 + pr] += retrace_cols(A[pr], a2, u, B[pr]);
+      }
+    }
+  }
+  block_sum_store<3>(v, part + 3 * lb);
+}
+
+// FP32 links of a shape the tiles do not divide: one probe at a time, the
+// traces from the rows of A u (again for the rounding of the step)
+__device__ __forceinline__ su3<double> promote(const su3<float> &m) {
+  su3<double> d;
+#pragma unroll
+  for (int k = 0; k < 9; k++) d.e[k] = mk<double>((double)m.e[k].re, (double)m.e[k].im);
+  return d;
+}
+__global__ __launch_bounds__(kBlock) void k_line_search_rows(const float2 *__restrict__ U, const float2 *__restrict__ F,
                                                        double *__restrict__ part, Geo g,
                                                        const Ctrl *__restrict__ ctrl, int force) {
   if (ctrl->done) return;
@@ -135,7 +228,7 @@ __global__ __launch_bounds__(kBlock) void k_line_search(const vec2<T> *__restric
 #pragma unroll 1
     for (int pr = 1; pr <= 2; pr++) {
       const double al = pr == 1 ? 0.15 : 0.30;
-      const su3<double> A = gauge_at64<T>(F, V, i, al);
+      const su3<double> A = gauge_at64<float>(F, V, i, al);
       double acc = 0.0;
 #pragma unroll 1
       for (int mu = 0; mu < kND; mu++) {
@@ -143,175 +236,14 @@ __global__ __launch_bounds__(kBlock) void k_line_search(const vec2<T> *__restric
         // matrix is built, which keeps the register peak lower
         cx<double> au[6];
         {
-          const su3<double> u = promote<T>(load_link<T>(U, mu, i, V));
+          const su3<double> u = promote(load_link<float>(U, mu, i, V));
           if (pr == 1) v[0] += u.e[0].re + u.e[4].re + u.e[8].re;
           ab_rows01<double>(A, u, au);
         }
-        acc += retrace_rows01_dag<double>(au, gauge_at64<T>(F, V, nb_fwd(g, i, x, mu), al));
+        acc += retrace_rows01_dag<double>(au, gauge_at64<float>(F, V, nb_fwd(g, i, x, mu), al));
       }
       v[pr] = acc;
     }
-  }
-  block_sum_store<3>(v, part + 3 * lb);
-}
-
-// ---------------------------------------------------------------------------
-// The same probes with each probe matrix built once.  A workgroup owns a
-// TX x TY x TZ x TT tile of 256 sites and builds, per probe, the matrices
-// g(x; alpha) of its sites and of the forward faces of the tile (the
-// neighbours x + mu outside it) into LDS: 2 + 256 / TX + ... builds per
-// 256 sites instead of 5 per site.  Only columns 0 and 1 are kept: with
-// M = A u (columns 0, 1 from u's stored columns) and B the neighbour's
-// matrix, both in SU(3) so that their third columns are conj(c0 x c1),
-//   Re tr(A u B^dag) = Re q00 + Re q11 + Re(q00 q11 - q01 q10),
-//   q_jk = sum_r M_j[r] conj(B_k[r])
-// (the Binet-Cauchy identity for the third columns), so neither u's nor
-// B's third column is ever formed; the probe at 0 takes u's third diagonal
-// entry from the same identity.  HOLD keeps a site's link columns in
-// registers for both probes; without it they are loaded again for the
-// second probe (from the caches), which frees registers for more waves.
-// The arithmetic is FP64, as in k_line_search.
-// ---------------------------------------------------------------------------
-template <typename T, int TX, int TY, int TZ, int TT, bool HOLD>
-__global__ __launch_bounds__(kBlock) void k_line_search_tile(const vec2<T> *__restrict__ U,
-                                                            const vec2<T> *__restrict__ F, double *__restrict__ part,
-                                                            Geo g, const Ctrl *__restrict__ ctrl, int force) {
-  constexpr int NT = TX * TY * TZ * TT;
-  static_assert(NT == kBlock, "one site per thread");
-  constexpr int HX = TY * TZ * TT, HY = TX * TZ * TT, HZ = TX * TY * TT, HT = TX * TY * TZ;
-  constexpr int OX = NT, OY = OX + HX, OZ = OY + HY, OT = OZ + HZ, NB = OT + HT;
-  __shared__ double lds[12 * NB];  // entry e of slot j (re, im of 6 complex) at lds[e * NB + j]
-  if (ctrl->done) return;
-  if (!force && !(ctrl->theta > ctrl->cg_tol)) return;
-  const long long V = g.V;
-  const unsigned lb = logical_block(g);
-  const int ntx = g.L[0] / TX, nty = g.L[1] / TY, ntz = g.L[2] / TZ;
-  unsigned r = lb;
-  const int x0 = (int)(r % (unsigned)ntx) * TX;
-  r /= (unsigned)ntx;
-  const int y0 = (int)(r % (unsigned)nty) * TY;
-  r /= (unsigned)nty;
-  const int z0 = (int)(r % (unsigned)ntz) * TZ;
-  const int t0 = (int)(r / (unsigned)ntz) * TT;
-  const int tid = threadIdx.x;
-  const int lx = tid % TX, ly = (tid / TX) % TY, lz = (tid / (TX * TY)) % TZ, lt = tid / (TX * TY * TZ);
-  auto site = [&](int x, int y, int z, int t) -> long long {
-    return (long long)x + g.S[1] * y + g.S[2] * z + g.S[3] * t;
-  };
-  const long long me = site(x0 + lx, y0 + ly, z0 + lz, t0 + lt);
-  // LDS slot of the forward neighbour in each direction
-  int nbs[4];
-  nbs[0] = lx < TX - 1 ? tid + 1 : OX + ly + TY * (lz + TZ * lt);
-  nbs[1] = ly < TY - 1 ? tid + TX : OY + lx + TX * (lz + TZ * lt);
-  nbs[2] = lz < TZ - 1 ? tid + TX * TY : OZ + lx + TX * (ly + TY * lt);
-  nbs[3] = lt < TT - 1 ? tid + TX * TY * TZ : OT + lx + TX * (ly + TY * lz);
-  // this site's link columns (col 0 rows 0..2, col 1 rows 0..2)
-  cx<T> uh[HOLD ? kND : 1][6];
-  auto load_u = [&](int mu, cx<T> (&w)[6]) {
-#pragma unroll
-    for (int k = 0; k < 6; k++) w[k] = ld<T>(U + ((long long)mu * 6 + k) * V + me);
-  };
-  double v[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-  for (int mu = 0; mu < kND; mu++) {
-    cx<T> w[6];
-    load_u(mu, w);
-    if constexpr (HOLD) {
-#pragma unroll
-      for (int k = 0; k < 6; k++) uh[mu][k] = w[k];
-    }
-    const double u00r = w[0].re, u00i = w[0].im, u10r = w[1].re, u10i = w[1].im;
-    const double u01r = w[3].re, u01i = w[3].im, u11r = w[4].re, u11i = w[4].im;
-    // Re U00 + Re U11 + Re U22, U22 = conj(U00 U11 - U10 U01)
-    v[0] += u00r + u11r + (u00r * u11r - u00i * u11i) - (u10r * u01r - u10i * u01i);
-  }
-#pragma unroll 1
-  for (int pr = 1; pr <= 2; pr++) {
-    const double al = pr == 1 ? 0.15 : 0.30;
-    if (pr == 2) __syncthreads();  // the first probe's matrices are no longer read
-    for (int j = tid; j < NB; j += kBlock) {
-      long long s = me;
-      if (j >= NT) {
-        int h = j - NT;
-        if (h < HX) {
-          s = site((x0 + TX) % g.L[0], y0 + h % TY, z0 + (h / TY) % TZ, t0 + h / (TY * TZ));
-        } else if ((h -= HX) < HY) {
-          s = site(x0 + h % TX, (y0 + TY) % g.L[1], z0 + (h / TX) % TZ, t0 + h / (TX * TZ));
-        } else if ((h -= HY) < HZ) {
-          s = site(x0 + h % TX, y0 + (h / TX) % TY, (z0 + TZ) % g.L[2], t0 + h / (TX * TY));
-        } else {
-          h -= HZ;
-          s = site(x0 + h % TX, y0 + (h / TX) % TY, z0 + h / (TX * TY), (t0 + TT) % g.L[3]);
-        }
-      }
-      auto f = [&](long long k) {
-        const cx<T> z = ld<T>(F + k * V + s);
-        return mk<double>((double)z.re, (double)z.im);
-      };
-      const su3<double> m = gauge_cols01<double>(f(0), f(1), f(2), f(3), al);
-      const cx<double> c[6] = {m.e[0], m.e[3], m.e[6], m.e[1], m.e[4], m.e[7]};
-#pragma unroll
-      for (int e = 0; e < 6; e++) {
-        lds[(2 * e) * NB + j] = c[e].re;
-        lds[(2 * e + 1) * NB + j] = c[e].im;
-      }
-    }
-    __syncthreads();
-    // this site's matrix A, completed: a[r][k] = A_rk
-    cx<double> a[3][3];
-#pragma unroll
-    for (int rr = 0; rr < 3; rr++)
-#pragma unroll
-      for (int k = 0; k < 2; k++)
-        a[rr][k] = mk<double>(lds[(2 * (3 * k + rr)) * NB + tid], lds[(2 * (3 * k + rr) + 1) * NB + tid]);
-    a[0][2] = cconj(csub(cmul(a[1][0], a[2][1]), cmul(a[2][0], a[1][1])));
-    a[1][2] = cconj(csub(cmul(a[2][0], a[0][1]), cmul(a[0][0], a[2][1])));
-    a[2][2] = cconj(csub(cmul(a[0][0], a[1][1]), cmul(a[1][0], a[0][1])));
-    // one direction's trace: nb is the LDS slot of the forward neighbour
-    auto trace_mu = [&](int mu, int nb) -> double {
-      cx<T> w[6];
-      if constexpr (HOLD) {
-#pragma unroll
-        for (int k = 0; k < 6; k++) w[k] = uh[mu][k];
-      } else {
-        load_u(mu, w);
-      }
-      // M = A u, columns 0 and 1
-      cx<double> M[2][3];
-#pragma unroll
-      for (int jc = 0; jc < 2; jc++) {
-        const cx<double> u0 = mk<double>((double)w[3 * jc].re, (double)w[3 * jc].im);
-        const cx<double> u1 = mk<double>((double)w[3 * jc + 1].re, (double)w[3 * jc + 1].im);
-        const cx<double> u2 = mk<double>((double)w[3 * jc + 2].re, (double)w[3 * jc + 2].im);
-#pragma unroll
-        for (int rr = 0; rr < 3; rr++)
-          M[jc][rr] = cadd(cadd(cmul(a[rr][0], u0), cmul(a[rr][1], u1)), cmul(a[rr][2], u2));
-      }
-      cx<double> q[2][2];
-#pragma unroll
-      for (int k = 0; k < 2; k++) {
-        cx<double> bk[3];
-#pragma unroll
-        for (int rr = 0; rr < 3; rr++)
-          bk[rr] = mk<double>(lds[(2 * (3 * k + rr)) * NB + nb], lds[(2 * (3 * k + rr) + 1) * NB + nb]);
-#pragma unroll
-        for (int jc = 0; jc < 2; jc++)
-          q[jc][k] = cadd(cadd(cmulc(M[jc][0], bk[0]), cmulc(M[jc][1], bk[1])), cmulc(M[jc][2], bk[2]));
-      }
-      const cx<double> d = csub(cmul(q[0][0], q[1][1]), cmul(q[0][1], q[1][0]));
-      return q[0][0].re + q[1][1].re + d.re;
-    };
-    double acc = 0.0;
-    if constexpr (HOLD) {
-#pragma unroll
-      for (int mu = 0; mu < kND; mu++) acc += trace_mu(mu, nbs[mu]);
-    } else {
-      // one direction at a time: fewer values live
-#pragma unroll 1
-      for (int mu = 0; mu < kND; mu++)
-        acc += trace_mu(mu, mu == 0 ? nbs[0] : mu == 1 ? nbs[1] : mu == 2 ? nbs[2] : nbs[3]);
-    }
-    v[pr] = acc;
   }
   block_sum_store<3>(v, part + 3 * lb);
 }
@@ -747,37 +679,22 @@ template <typename T> void launch_copy(const void *F, void *a, long long V, cons
   const unsigned b = (unsigned)std::min<long long>(nblk(n4), 8192);
   hipLaunchKernelGGL(k_copy<T>, dim3(b), dim3(kBlock), 0, s, (const vec2<T> *)F, (vec2<T> *)a, n4, ctrl);
 }
-template <typename T, int TX, int TY, int TZ, int TT, bool HOLD>
-static void launch_ls_tile(const void *U, const void *F, double *part, Geo g, const Ctrl *ctrl, int force,
-                           hipStream_t s) {
-  g.xcd = g.xcd ? 1 : 0;  // tiles are numbered x fastest: plain or XCD-contiguous
-  hipLaunchKernelGGL((k_line_search_tile<T, TX, TY, TZ, TT, HOLD>), dim3(nblk(g.V)), dim3(kBlock), 0, s,
-                     (const vec2<T> *)U, (const vec2<T> *)F, part, g, ctrl, force);
-}
-
-bool ls_tile_fits(const Geo &g, int tile) {
-  if (tile < 1 || tile > kLsTiles) return false;
-  const int *t = kLsTileShape[tile - 1];
-  for (int mu = 0; mu < 4; mu++)
-    if (g.L[mu] % t[mu]) return false;
-  return true;
-}
-
 template <typename T>
 void launch_line_search(const void *U, const void *F, double *part, const Geo &g, const Ctrl *ctrl, int force,
-                        hipStream_t s, int tile) {
-  switch (ls_tile_fits(g, tile) ? tile : 0) {
-    case 1: return launch_ls_tile<T, 8, 4, 4, 2, true>(U, F, part, g, ctrl, force, s);
-    case 2: return launch_ls_tile<T, 4, 4, 4, 4, true>(U, F, part, g, ctrl, force, s);
-    case 3: return launch_ls_tile<T, 8, 8, 2, 2, true>(U, F, part, g, ctrl, force, s);
-    case 4: return launch_ls_tile<T, 16, 4, 2, 2, true>(U, F, part, g, ctrl, force, s);
-    case 5: return launch_ls_tile<T, 8, 4, 4, 2, false>(U, F, part, g, ctrl, force, s);
-    case 6: return launch_ls_tile<T, 4, 4, 4, 4, false>(U, F, part, g, ctrl, force, s);
-    case 7: return launch_ls_tile<T, 8, 8, 2, 2, false>(U, F, part, g, ctrl, force, s);
-    case 8: return launch_ls_tile<T, 16, 4, 2, 2, false>(U, F, part, g, ctrl, force, s);
-    default:
-      hipLaunchKernelGGL(k_line_search<T>, dim3(nblk(g.V)), dim3(kBlock), 0, s, (const vec2<T> *)U,
-                         (const vec2<T> *)F, part, g, ctrl, force);
+                        hipStream_t s) {
+  if constexpr (sizeof(T) == 4) {
+    Geo gt = g;
+    if (g.L[0] % 8 || g.L[1] % 4 || g.L[2] % 4 || g.L[3] % 2) {
+      hipLaunchKernelGGL(k_line_search_rows, dim3(nblk(g.V)), dim3(kBlock), 0, s, (const float2 *)U,
+                         (const float2 *)F, part, g, ctrl, force);
+      return;
+    }
+    gt.xcd = g.xcd ? 1 : 0;  // tiles are numbered x fastest: plain or XCD-contiguous
+    hipLaunchKernelGGL(k_line_search<T>, dim3(nblk(g.V)), dim3(kBlock), 0, s, (const vec2<T> *)U,
+                       (const vec2<T> *)F, part, gt, ctrl, force);
+  } else {
+    hipLaunchKernelGGL(k_line_search<T>, dim3(nblk(g.V)), dim3(kBlock), 0, s, (const vec2<T> *)U,
+                       (const vec2<T> *)F, part, g, ctrl, force);
   }
 }
 template <typename T>
@@ -809,7 +726,7 @@ template <typename T> void launch_identity(void *G, long long V, hipStream_t s) 
   template void launch_cg_update<T>(const void *, void *, long long, const Ctrl *, hipStream_t);               \
   template void launch_copy<T>(const void *, void *, long long, const Ctrl *, hipStream_t);                    \
   template void launch_line_search<T>(const void *, const void *, double *, const Geo &, const Ctrl *, int,   \
-                                      hipStream_t, int);                                                      \
+                                      hipStream_t);                                                           \
   template void launch_egauge<T>(void *, const void *, void *, const Geo &, const Ctrl *, int, hipStream_t);  \
   template void launch_egauge_deriv<T>(const void *, void *, const void *, void *, void *, void *, double *,     \
                                        const Geo &, const Ctrl *, hipStream_t);                                   \

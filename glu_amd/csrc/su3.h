@@ -156,6 +156,65 @@ __device__ __forceinline__ su3<T> gauge_cols01(cx<T> f0, cx<T> f1, cx<T> f2, cx<
   return g;
 }
 
+// The packed direction at one site, ready to give gauge_matrix's columns at
+// any step.  With v0 = e0 + alpha x0, v1 = e1 + alpha x1 the raw columns of
+// 1 + alpha X, the terms linear in alpha cancel in every product the
+// Gram-Schmidt needs, |v0|^2 = 1 + alpha^2 s00, |v1|^2 = 1 + alpha^2 s11 and
+// <v0, v1> = alpha^2 s01, so a second step costs two square roots and the
+// scaling only (and the two columns are as orthogonal as the sums allow)
+struct ProbeSite {
+  cx<double> f0, f1, f2, f3, s01;
+  double s00, s11;
+  __device__ __forceinline__ void set(cx<double> a, cx<double> b, cx<double> c, cx<double> d) {
+    f0 = a, f1 = b, f2 = c, f3 = d;
+    const double n1 = cnorm2(f1), w = f0.re - f0.im;
+    s00 = f0.im * f0.im + n1 + cnorm2(f2);
+    s11 = f0.re * f0.re + n1 + cnorm2(f3);
+    s01 = cmulc(f2, f3);
+    s01.re -= f1.im * w;
+    s01.im += f1.re * w;
+  }
+  // columns 0 and 1 of P(1 + alpha X): c[0..2], c[3..5]
+  __device__ __forceinline__ void cols(double al, cx<double> (&c)[6]) const {
+    const double a2 = al * al;
+    const double n0 = rsqrt_nr(1.0 + a2 * s00), m0 = n0 * al;
+    const double t = n0 * a2;  // <c0, v1> = t s01
+    const double n1 = rsqrt_nr(1.0 + a2 * s11 - t * t * cnorm2(s01)), m1 = n1 * al;
+    c[0] = mk<double>(n0, m0 * f0.im);
+    c[1] = mk<double>(-m0 * f1.re, m0 * f1.im);
+    c[2] = mk<double>(-m0 * f2.re, m0 * f2.im);
+    const cx<double> p = cscale(s01, n1 * t);
+    c[3] = csub(cscale(f1, m1), cmul(p, c[0]));
+    c[4] = csub(mk<double>(n1, -m1 * f0.re), cmul(p, c[1]));
+    c[5] = csub(mk<double>(-m1 * f3.re, m1 * f3.im), cmul(p, c[2]));
+  }
+};
+
+// Re tr(A u B^dagger) for SU(3) matrices given by their columns 0 and 1
+// (c[0..2], c[3..5]; the third column of each is conj(col0 x col1)), a2 the
+// third column of A.  With M = A u and q_jk = sum_r M_j[r] conj(B_k[r]) the
+// third columns enter through the Binet-Cauchy identity as
+// Re(q00 q11 - q01 q10): neither u's nor B's is formed.
+__device__ __forceinline__ cx<double> third(cx<double> a, cx<double> b, cx<double> c, cx<double> d) {
+  return cconj(csub(cmul(a, d), cmul(b, c)));  // conj(a d - b c)
+}
+__device__ __forceinline__ double retrace_cols(const cx<double> (&A)[6], const cx<double> (&a2)[3],
+                                               const cx<double> (&u)[6], const cx<double> (&B)[6]) {
+  cx<double> q[2][2];
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    cx<double> M[3];
+#pragma unroll
+    for (int r = 0; r < 3; r++)
+      M[r] = cadd(cadd(cmul(A[r], u[3 * j]), cmul(A[3 + r], u[3 * j + 1])), cmul(a2[r], u[3 * j + 2]));
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+      q[j][k] = cadd(cadd(cmulc(M[0], B[3 * k]), cmulc(M[1], B[3 * k + 1])), cmulc(M[2], B[3 * k + 2]));
+  }
+  const cx<double> d = csub(cmul(q[0][0], q[1][1]), cmul(q[0][1], q[1][0]));
+  return q[0][0].re + q[1][1].re + d.re;
+}
+
 // b <- a b c^dagger with columns 0,1 of the product and column 2 completed:
 // Gfix/gtrans.c:32-141
 template <typename T>
