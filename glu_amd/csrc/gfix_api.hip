@@ -336,7 +336,7 @@ int upload_links(glu_gfix_ctx *c, SiteGather gather, void *arg) {
             hipSuccess ||
         hipEventRecord(c->hev[b], c->stream) != hipSuccess)
       return gfix_fail(-2, "link upload failed");
-    launch_pack<double>((const double *)c->stage, c->U64, V, 4, s0, n, c->stream);
+    launch_pack((const double *)c->stage, c->U64, V, s0, n, c->stream);
   }
   if (hipStreamSynchronize(c->stream) != hipSuccess) return gfix_fail(-2, "link upload: %s", "sync failed");
   return 0;
@@ -357,7 +357,7 @@ int download_links(glu_gfix_ctx *c, SiteScatter scatter, void *arg) {
   for (long long s0 = 0; s0 < V; s0 += kHostChunk, k++) {
     const long long n = std::min(kHostChunk, V - s0);
     const int b = k & 1;
-    launch_unpack<double>(c->U64, (double *)c->stage, V, 4, s0, n, c->stream);
+    launch_unpack(c->U64, (double *)c->stage, V, s0, n, c->stream);
     if (hipMemcpyAsync(c->hstage[b], c->stage, (size_t)n * 72 * sizeof(double), hipMemcpyDeviceToHost, c->stream) !=
             hipSuccess ||
         hipEventRecord(c->hev[b], c->stream) != hipSuccess)
@@ -395,14 +395,14 @@ extern "C" int glu_gfix_get_links(glu_gfix_ctx *c, double *links) {
 
 extern "C" int glu_gfix_set_links_device(glu_gfix_ctx *c, const double *links_dev) {
   if (!c || !links_dev) return gfix_fail(-1, "glu_gfix_set_links_device: null argument");
-  launch_pack<double>(links_dev, c->U64, c->g.V, 4, 0, c->g.V, c->stream);
+  launch_pack(links_dev, c->U64, c->g.V, 0, c->g.V, c->stream);
   if (hipStreamSynchronize(c->stream) != hipSuccess) return gfix_fail(-2, "pack failed");
   return 0;
 }
 
 extern "C" int glu_gfix_get_links_device(glu_gfix_ctx *c, double *links_dev) {
   if (!c || !links_dev) return gfix_fail(-1, "glu_gfix_get_links_device: null argument");
-  launch_unpack<double>(c->U64, links_dev, c->g.V, 4, 0, c->g.V, c->stream);
+  launch_unpack(c->U64, links_dev, c->g.V, 0, c->g.V, c->stream);
   if (hipStreamSynchronize(c->stream) != hipSuccess) return gfix_fail(-2, "unpack failed");
   return 0;
 }

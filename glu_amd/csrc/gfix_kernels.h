@@ -72,10 +72,8 @@ void launch_egauge(void *U, const void *F, void *G, const Geo &g, const Ctrl *ct
 template <typename T>
 void launch_egauge_deriv(const void *Uin, void *Uout, const void *D, void *G, void *Fin, void *Fout, double *part,
                          const Geo &g, const Ctrl *ctrl, hipStream_t s);
-template <typename T>
-void launch_pack(const double *aos, void *U, long long V, int nd, long long site0, long long n, hipStream_t s);
-template <typename T>
-void launch_unpack(const void *U, double *aos, long long V, int nd, long long site0, long long n, hipStream_t s);
+void launch_pack(const double *aos, void *U, long long V, long long site0, long long n, hipStream_t s);
+void launch_unpack(const void *U, double *aos, long long V, long long site0, long long n, hipStream_t s);
 template <typename T> void launch_identity(void *G, long long V, hipStream_t s);
 
 void launch_fin_theta(const double *part, long long nb, Ctrl *ctrl, double norm, hipStream_t s);

@@ -113,7 +113,7 @@ extern "C" int glu_gfix_write_nersc(glu_gfix_ctx *c, const char *path, int two_r
   int rc = 0;
   for (long long s0 = 0; s0 < V && !rc; s0 += kChunk) {
     const long long n = std::min(kChunk, V - s0);
-    launch_unpack<double>(c->U64, (double *)c->stage, V, 4, s0, n, c->stream);
+    launch_unpack(c->U64, (double *)c->stage, V, s0, n, c->stream);
     if (hipMemcpyAsync(h.data(), c->stage, (size_t)n * 72 * sizeof(double), hipMemcpyDeviceToHost, c->stream) !=
             hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess) {

@@ -234,7 +234,7 @@ int start(glu_gfix_server *s, Request &r, bool *finished) {
   if (r.switch_theta > 0.0) c->switch_theta = r.switch_theta;
   c->mwc_live = 0;  // a pooled context's streams never carry over
   c->rng_seed = r.seed ? r.seed : 1;
-  launch_pack<double>(r.links, c->U64, c->g.V, 4, 0, c->g.V, c->stream);
+  launch_pack(r.links, c->U64, c->g.V, 0, c->g.V, c->stream);
   if (r.random_transform) {  // GLU's read_and_fix with RANDOM_TRANSFORM = YES
     if (int rc = mwc_seed(c, c->rng_seed, c->rng_threads)) return rc;
     if (int rc = mwc_random_transform(c)) return rc;
@@ -292,7 +292,7 @@ int after_attempt(Request &r, size_t loc, double theta) {
   // under random_transform drawn from GLU's streams, seeded with the
   // request's seed at its first restart as glu_gfix_landau does (a pooled
   // context's streams never carry over from another request)
-  launch_pack<double>(r.links, c->U64, c->g.V, 4, 0, c->g.V, c->stream);
+  launch_pack(r.links, c->U64, c->g.V, 0, c->g.V, c->stream);
   if (r.attempt == 1 && !r.random_transform)
     if (int rc = mwc_seed(c, (uint32_t)(r.restart_seed ? r.restart_seed : 1), c->rng_threads)) return rc;
   if (int rc = mwc_random_transform(c)) return rc;
@@ -306,7 +306,7 @@ int after_run(Request &r) { return after_attempt(r, r.ctx->run.iters, r.ctx->run
 // enqueue the copy of the fixed links into the request's buffer
 int copy_out(Request &r) {
   glu_gfix_ctx *c = r.ctx;
-  launch_unpack<double>(c->U64, r.links, c->g.V, 4, 0, c->g.V, c->stream);
+  launch_unpack(c->U64, r.links, c->g.V, 0, c->g.V, c->stream);
   if (hipEventRecord(r.ev, c->stream) != hipSuccess) return gfix_fail(-2, "serving: event record failed");
   r.copying = 1;
   return 0;
