@@ -79,8 +79,11 @@ struct glu_gfix_ctx {
   int use_zt = 1;     // Landau: z and t axes with p^2 in one pass after the x-y pass
   int zt_pv = 0;      // x values per workgroup of that pass (variant, tuned)
   // workgroup order (Geo::xcd) of the derivative / fused update and of the
-  // line search; set by the autotuner
-  int ord_eg = 1, ord_ls = 1;
+  // line search; set by the autotuner.  Untuned, the FP64 update of 32^3x64
+  // takes 417 us in time slabs (2; 1 where they do not divide), 457
+  // contiguous and 473 plain, of 24^3x48 134, 138 and 153 us; the line
+  // search does not care
+  int ord_eg = 2, ord_ls = 1;
   int ord_cl = 1;  // Coulomb slice stencils: XCD-contiguous (1) or plain (0)
   int use_graph = 0;  // replay iteration batches from captured HIP graphs
   // iterations enqueued between host checks; the iterations enqueued past
