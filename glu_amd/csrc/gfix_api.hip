@@ -1052,18 +1052,13 @@ extern "C" int glu_gfix_mixed_split(glu_gfix_ctx *c, size_t *a, size_t *b) {
 // ---------------------------------------------------------------------------
 extern "C" int glu_gfix_measure(glu_gfix_ctx *c, double *plaq, double *tr, double *mx, double *func, double *tlink) {
   if (!c) return gfix_fail(-1, "null context");
-  launch_measure(c->U64, c->part, c->g, c->stream);
-  std::vector<double> h(c->nblk * 4);
-  if (hipMemcpyAsync(h.data(), c->part, h.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
+  double *out = c->part + 4 * c->nblk;  // spare slots after the partials
+  launch_measure(c->U64, c->part, out, geo_order(c, 1), c->stream);
+  double h[4];
+  if (hipMemcpyAsync(h, out, sizeof(h), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
       hipStreamSynchronize(c->stream) != hipSuccess)
     return gfix_fail(-2, "measure readback failed");
-  double p = 0, t = 0, tt = 0, m = -1e300;
-  for (long long b = 0; b < c->nblk; b++) {
-    p += h[4 * b];
-    t += h[4 * b + 1];
-    tt += h[4 * b + 2];
-    m = h[4 * b + 3] > m ? h[4 * b + 3] : m;
-  }
+  const double p = h[0], t = h[1], tt = h[2], m = h[3];
   const double V = (double)c->g.V;
   if (plaq) *plaq = 2.0 * p / (3.0 * 4 * 3 * V);
   if (tr) *tr = t / (4 * 3 * V);

@@ -89,6 +89,8 @@ void launch_demote(const void *U, void *W, long long n, hipStream_t s);
 void launch_apply_gauge(void *U, const void *G, const Geo &g, hipStream_t s);
 void launch_promote(const void *a, void *b, long long n, hipStream_t s);
 void launch_reunit(void *U, long long V, int nd, hipStream_t s);
-void launch_measure(const void *U, double *part, const Geo &g, hipStream_t s);
+// the plaquette, link-trace and temporal-trace sums and the largest link
+// trace of the links go to out[0..4)
+void launch_measure(const void *U, double *part, double *out, const Geo &g, hipStream_t s);
 
 }  // namespace gfix

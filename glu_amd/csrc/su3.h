@@ -190,29 +190,49 @@ struct ProbeSite {
   }
 };
 
-// Re tr(A u B^dagger) for SU(3) matrices given by their columns 0 and 1
-// (c[0..2], c[3..5]; the third column of each is conj(col0 x col1)), a2 the
-// third column of A.  With M = A u and q_jk = sum_r M_j[r] conj(B_k[r]) the
-// third columns enter through the Binet-Cauchy identity as
-// Re(q00 q11 - q01 q10): neither u's nor B's is formed.
+// conj(a d - b c): an entry of a third column from two rows of the others
 __device__ __forceinline__ cx<double> third(cx<double> a, cx<double> b, cx<double> c, cx<double> d) {
-  return cconj(csub(cmul(a, d), cmul(b, c)));  // conj(a d - b c)
+  return cconj(csub(cmul(a, d), cmul(b, c)));
 }
-__device__ __forceinline__ double retrace_cols(const cx<double> (&A)[6], const cx<double> (&a2)[3],
-                                               const cx<double> (&u)[6], const cx<double> (&B)[6]) {
-  cx<double> q[2][2];
+// columns 0 and 1 (m[0..2], m[3..5]) of A u: A by its columns 0, 1 and its
+// third a2, u by its columns 0 and 1
+__device__ __forceinline__ void mul_cols01(const cx<double> (&A)[6], const cx<double> (&a2)[3],
+                                           const cx<double> (&u)[6], cx<double> (&m)[6]) {
 #pragma unroll
-  for (int j = 0; j < 2; j++) {
-    cx<double> M[3];
+  for (int j = 0; j < 2; j++)
 #pragma unroll
     for (int r = 0; r < 3; r++)
-      M[r] = cadd(cadd(cmul(A[r], u[3 * j]), cmul(A[3 + r], u[3 * j + 1])), cmul(a2[r], u[3 * j + 2]));
+      m[3 * j + r] = cadd(cadd(cmul(A[r], u[3 * j]), cmul(A[3 + r], u[3 * j + 1])), cmul(a2[r], u[3 * j + 2]));
+}
+// Re tr(M B^dagger) of two SU(3) matrices given by columns 0 and 1: with
+// q_jk = sum_r M_j[r] conj(B_k[r]) the third columns, conj(col0 x col1) of
+// each, enter through the Binet-Cauchy identity as Re(q00 q11 - q01 q10), so
+// neither is formed
+__device__ __forceinline__ double retrace_cols(const cx<double> (&M)[6], const cx<double> (&B)[6]) {
+  cx<double> q[2][2];
+#pragma unroll
+  for (int j = 0; j < 2; j++)
 #pragma unroll
     for (int k = 0; k < 2; k++)
-      q[j][k] = cadd(cadd(cmulc(M[0], B[3 * k]), cmulc(M[1], B[3 * k + 1])), cmulc(M[2], B[3 * k + 2]));
-  }
+      q[j][k] = cadd(cadd(cmulc(M[3 * j], B[3 * k]), cmulc(M[3 * j + 1], B[3 * k + 1])),
+                     cmulc(M[3 * j + 2], B[3 * k + 2]));
   const cx<double> d = csub(cmul(q[0][0], q[1][1]), cmul(q[0][1], q[1][0]));
   return q[0][0].re + q[1][1].re + d.re;
+}
+// the two stored columns of a link, as they are
+template <typename T>
+__device__ __forceinline__ void load_cols(const vec2<T> *__restrict__ U, int mu, long long i, long long V,
+                                          cx<double> (&u)[6]) {
+#pragma unroll
+  for (int k = 0; k < 6; k++) {
+    const cx<T> w = ld<T>(U + ((long long)mu * 6 + k) * V + i);
+    u[k] = mk<double>((double)w.re, (double)w.im);
+  }
+}
+__device__ __forceinline__ void third_col(const cx<double> (&a)[6], cx<double> (&a2)[3]) {
+  a2[0] = third(a[1], a[2], a[4], a[5]);
+  a2[1] = third(a[2], a[0], a[5], a[3]);
+  a2[2] = third(a[0], a[1], a[3], a[4]);
 }
 
 // b <- a b c^dagger with columns 0,1 of the product and column 2 completed:
