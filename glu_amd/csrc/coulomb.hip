@@ -106,13 +106,29 @@ __device__ __forceinline__ void herm_short(const su3<double> &U, double s[10]) {
   s[9] = 0.5 * (U.e[7].re - U.e[5].re);
 }
 
-// derivative of the gauge-rotated spatial links: Gfix/CFACG.c:92-163
+// the end of iteration n of a running slice (every running slice of a call
+// has made the same number): count and stop test (Gfix/CFACG.c:366-382)
+__device__ __forceinline__ bool slice_stops(const SliceCtrl &sc, int t, long long n) {
+  return n > 0 && !(sc.theta[t] > sc.acc && n < sc.max_iters);
+}
+__device__ __forceinline__ void slice_stop(const SliceCtrl &sc, int t, long long n) {
+  sc.iters[t] = n;
+  sc.done[t] = 1;
+}
+
+// derivative of the gauge-rotated spatial links: Gfix/CFACG.c:92-163.  The
+// stop test of the n iterations made so far comes first: every block of the
+// slice finds the same answer, its first block records it
 __global__ __launch_bounds__(kBlock) void k_cderiv(const double2 *__restrict__ U, const double2 *__restrict__ G,
-                                                  double2 *__restrict__ F, Geo g, SliceCtrl sc) {
+                                                  double2 *__restrict__ F, Geo g, SliceCtrl sc, long long n) {
   int t;
   long long bx;
   slice_block(g, sc, t, bx);
   if (sc.done[t]) return;
+  if (slice_stops(sc, t, n)) {
+    if (bx == 0 && threadIdx.x == 0) slice_stop(sc, t, n);
+    return;
+  }
   const long long xl = bx * blockDim.x + threadIdx.x;
   if (xl >= g.Lcu) return;
   const long long i = site_of(g, t, xl), V = g.V;
@@ -180,8 +196,50 @@ __device__ double block_reduce_1024(double v, double *sh) {
   return s;
 }
 
-// per-slice finaliser of the PR sums.  mode 0: SD start (inold, theta);
-// mode 1: loop iteration (theta, beta, inold) -- Gfix/CFACG.c:311-339
+// Slices of few blocks (kFuseBlocks) need no finaliser launches: every block
+// of the next kernel adds the slice's partial rows itself, in one order, and
+// the slice's first block writes the scalars.  On 16^3 slices (16 blocks)
+// the finalisers took 4 and 5 us of an iteration's 95; on 48^3 (432) the
+// repeated sums would cost more than the 6 us launches they replace.
+constexpr long long kFuseBlocks = 64;
+template <int NV>
+__device__ __forceinline__ void slice_sums(const double *__restrict__ part, int t, long long nbs, double (&s)[NV]) {
+  __shared__ double sh[NV][kBlock / kWave];
+  double v[NV];
+#pragma unroll
+  for (int j = 0; j < NV; j++) v[j] = 0.0;
+  for (long long k = threadIdx.x; k < nbs; k += kBlock)
+#pragma unroll
+    for (int j = 0; j < NV; j++) v[j] += part[NV * (t * nbs + k) + j];
+#pragma unroll
+  for (int j = 0; j < NV; j++) {
+    const double w = wave_sum(v[j]);
+    if (threadIdx.x % kWave == 0) sh[j][threadIdx.x / kWave] = w;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NV; j++) {
+    s[j] = 0.0;
+    for (int w = 0; w < kBlock / kWave; w++) s[j] += sh[j][w];
+  }
+}
+
+// theta and beta of a slice from its PR sums.  mode 0: SD start; mode 1: loop
+// iteration -- Gfix/CFACG.c:311-339.  insum becomes inold once every reader
+// of the old one is done (k_cfin_pr, or the line search that follows)
+__device__ __forceinline__ double pr_beta(const SliceCtrl &sc, int t, double s1, double s2, int mode) {
+  if (mode == 0) return 0.0;
+  double beta = s2 / sc.inold[t];
+  if (beta < 0.0) beta = 0.0;
+  if (s1 * sc.norm < sc.cg_tol) beta = s1 / sc.inold[t];
+  return beta;
+}
+__device__ __forceinline__ void pr_record(const SliceCtrl &sc, int t, double s1, double s2, double beta) {
+  sc.theta[t] = s1 * sc.norm;
+  sc.insum[t] = s1;
+  sc.sconj[t] = s2;
+  sc.beta[t] = beta;
+}
 __global__ void k_cfin_pr(const double *__restrict__ part, long long nbs, SliceCtrl sc, int mode) {
   const int t = blockIdx.x;
   if (sc.done[t]) return;
@@ -192,37 +250,33 @@ __global__ void k_cfin_pr(const double *__restrict__ part, long long nbs, SliceC
     b += part[2 * (t * nbs + k) + 1];
   }
   const double s1 = block_reduce_1024(a, sh), s2 = block_reduce_1024(b, sh);
-  if (threadIdx.x == 0) {
-    sc.theta[t] = s1 * sc.norm;
-    if (mode == 0) {
-      sc.inold[t] = s1;
-      sc.beta[t] = 0.0;
-    } else {
-      double beta = s2 / sc.inold[t];
-      if (beta < 0.0) beta = 0.0;
-      if (sc.theta[t] < sc.cg_tol) beta = s1 / sc.inold[t];
-      sc.inold[t] = s1;
-      sc.insum[t] = s1;
-      sc.sconj[t] = s2;
-      sc.beta[t] = beta;
-    }
-  }
+  if (threadIdx.x == 0) pr_record(sc, t, s1, s2, pr_beta(sc, t, s1, s2, mode));
 }
 
 // sn = in + beta sn (mode 1, Gfix/CFACG.c:359-365) or sn = in (mode 0, the
 // SD start, :323).  GLU's copy old = in is not made: the host swaps its in
 // and in_old pointers after every CG iteration, so the next derivative
 // lands in the old buffer and this iteration's in becomes in_old in place.
+// fuse: beta comes from the PR partials here
 __global__ __launch_bounds__(kBlock) void k_cupdate(const double2 *__restrict__ F, double2 *__restrict__ sn, Geo g,
-                                                   SliceCtrl sc, int mode) {
+                                                   SliceCtrl sc, int mode, const double *__restrict__ part,
+                                                   long long nbs, int fuse) {
   int t;
   long long bx;
   slice_block(g, sc, t, bx);
   if (sc.done[t]) return;
+  double beta;
+  if (fuse) {
+    double s[2];
+    slice_sums<2>(part, t, nbs, s);
+    beta = pr_beta(sc, t, s[0], s[1], mode);
+    if (bx == 0 && threadIdx.x == 0) pr_record(sc, t, s[0], s[1], beta);
+  } else {
+    beta = sc.beta[t];
+  }
   const long long xl = bx * blockDim.x + threadIdx.x;
   if (xl >= g.Lcu) return;
   const long long i = site_of(g, t, xl), V = g.V;
-  const double beta = mode ? sc.beta[t] : 0.0;
   for (int f = 0; f < 4; f++) {
     const double2 a = F[f * V + i];
     if (mode) {
@@ -249,6 +303,7 @@ __global__ __launch_bounds__(kBlock) void k_cline(const double2 *__restrict__ U,
   long long bx;
   slice_block(g, sc, t, bx);
   if (sc.done[t]) return;
+  if (bx == 0 && threadIdx.x == 0) sc.inold[t] = sc.insum[t];  // beta has been taken
   if (!force && !(sc.theta[t] > sc.cg_tol)) return;
   const long long xl = bx * blockDim.x + threadIdx.x;
   double v[3] = {0.0, 0.0, 0.0};
@@ -288,12 +343,30 @@ __device__ __forceinline__ double approx_min(const double al[3], const double f[
   return sol;
 }
 
-// step of each slice: parabola vertex (Gfix/line_search.c:118-138) or
-// GF_TUNE below CG_TOL / for FASD
+// step of a slice from its probe sums: parabola vertex
+// (Gfix/line_search.c:118-138) or GF_TUNE below CG_TOL / for FASD
+__device__ __forceinline__ bool ls_runs(const SliceCtrl &sc, int t, int force, int fixed) {
+  return !fixed && (force || (sc.theta[t] > sc.cg_tol));
+}
+__device__ __forceinline__ double ls_step(const SliceCtrl &sc, const double (&s)[3], bool do_ls) {
+  const double al[3] = {0.0, PC1, PC2};
+  const double val[3] = {-s[0], -s[1], -s[2]};
+  return do_ls ? approx_min(al, val) : sc.gf_alpha;
+}
+__device__ __forceinline__ void ls_record(const SliceCtrl &sc, int t, const double (&s)[3], double alpha, bool do_ls,
+                                          int force, int fixed) {
+  if (do_ls)
+    for (int j = 0; j < 3; j++) sc.probe[3 * t + j] = s[j];
+  sc.alpha[t] = alpha;
+  sc.did_ls[t] = do_ls;
+  // FACG row: theta measured before the step, the step, beta (0 at the
+  // SD start); FASD rows are written once theta is known (k_cfin_der)
+  if (!fixed) slice_rec(sc, t, sc.theta[t], alpha, force ? 0.0 : sc.beta[t]);
+}
 __global__ void k_cfin_ls(const double *__restrict__ part, long long nbs, SliceCtrl sc, int force, int fixed) {
   const int t = blockIdx.x;
   if (sc.done[t]) return;
-  const int do_ls = !fixed && (force || (sc.theta[t] > sc.cg_tol));
+  const bool do_ls = ls_runs(sc, t, force, fixed);
   __shared__ double sh[16];
   double s[3] = {0, 0, 0};
   if (do_ls) {
@@ -302,34 +375,32 @@ __global__ void k_cfin_ls(const double *__restrict__ part, long long nbs, SliceC
       for (int j = 0; j < 3; j++) a[j] += part[3 * (t * nbs + k) + j];
     for (int j = 0; j < 3; j++) s[j] = block_reduce_1024(a[j], sh);
   }
-  if (threadIdx.x == 0) {
-    if (do_ls) {
-      const double al[3] = {0.0, PC1, PC2};
-      const double val[3] = {-s[0], -s[1], -s[2]};
-      for (int j = 0; j < 3; j++) sc.probe[3 * t + j] = s[j];
-      sc.alpha[t] = approx_min(al, val);
-      sc.did_ls[t] = 1;
-    } else {
-      sc.alpha[t] = sc.gf_alpha;
-      sc.did_ls[t] = 0;
-    }
-    // FACG row: theta measured before the step, the step, beta (0 at the
-    // SD start); FASD rows are written once theta is known (k_cfin_der)
-    if (!fixed) slice_rec(sc, t, sc.theta[t], sc.alpha[t], force ? 0.0 : sc.beta[t]);
-  }
+  if (threadIdx.x == 0) ls_record(sc, t, s, ls_step(sc, s, do_ls), do_ls, force, fixed);
 }
 
-// G(x) <- P(1 + alpha_t X(F(x))) G(x): Gfix/line_search.c:101-115
+// G(x) <- P(1 + alpha_t X(F(x))) G(x): Gfix/line_search.c:101-115.  fuse: the
+// step comes from the probe partials here
 __global__ __launch_bounds__(kBlock) void k_cexp(double2 *__restrict__ G, const double2 *__restrict__ F, Geo g,
-                                                SliceCtrl sc) {
+                                                SliceCtrl sc, const double *__restrict__ part, long long nbs, int force,
+                                                int fuse) {
   int t;
   long long bx;
   slice_block(g, sc, t, bx);
   if (sc.done[t]) return;
+  double alpha;
+  if (fuse) {
+    const bool do_ls = ls_runs(sc, t, force, 0);
+    double s[3] = {0.0, 0.0, 0.0};
+    if (do_ls) slice_sums<3>(part, t, nbs, s);
+    alpha = ls_step(sc, s, do_ls);
+    if (bx == 0 && threadIdx.x == 0) ls_record(sc, t, s, alpha, do_ls, force, 0);
+  } else {
+    alpha = sc.alpha[t];
+  }
   const long long xl = bx * blockDim.x + threadIdx.x;
   if (xl >= g.Lcu) return;
   const long long i = site_of(g, t, xl), V = g.V;
-  const su3<double> a = cgauge_at(F, V, i, sc.alpha[t]);
+  const su3<double> a = cgauge_at(F, V, i, alpha);
   store_link<double>(G, 0, i, V, mul_cols<double>(a, load_link<double>(G, 0, i, V)));
 }
 
@@ -347,12 +418,10 @@ __global__ void k_cfin_der(const double *__restrict__ part, long long nbs, Slice
   }
 }
 
-__global__ void k_citer_end(SliceCtrl sc) {
-  for (int t = threadIdx.x; t < sc.T; t += blockDim.x) {
-    if (sc.done[t]) continue;
-    sc.iters[t]++;
-    if (!(sc.theta[t] > sc.acc && sc.iters[t] < sc.max_iters)) sc.done[t] = 1;
-  }
+// the stop test after the last iteration of a batch
+__global__ void k_cstop(SliceCtrl sc, long long n) {
+  for (int t = threadIdx.x; t < sc.T; t += blockDim.x)
+    if (!sc.done[t] && slice_stops(sc, t, n)) slice_stop(sc, t, n);
 }
 
 // reunitarise the slice transforms and record the largest |sum |g|^2 - NC|
@@ -514,41 +583,41 @@ static int run_slices(glu_gfix_ctx *c, int method, const std::vector<int> &activ
   double2 *U = (double2 *)c->U64, *G = (double2 *)cs->G, *F = (double2 *)c->F, *sn = (double2 *)c->sn,
           *O = (double2 *)c->old;
   double *part = c->part;
-  if (method == GLU_GFIX_CG) {
-    // SD start: derivative, FA, theta and inold, line search, sn = in; the
-    // pointer swap makes in the in_old of the first CG iteration.  The CG
-    // state lives within this call (every call starts with an SD step), so
-    // a slice that stopped may keep its fields in either buffer.
-    GFIX_PROF(c, PK_CDERIV, hipLaunchKernelGGL(k_cderiv, grid, blk, 0, s, U, G, F, g, sc));
+  const int fuse = cs->nbs <= kFuseBlocks;
+  long long n = 0;  // iterations made
+  // one FACG step: derivative, FA, theta and beta, direction, line search,
+  // transform; mode 0 is the SD start (sn = in), whose in becomes the in_old
+  // of the first CG iteration by the pointer swap.  The CG state lives
+  // within this call (every call starts with an SD step), so a slice that
+  // stopped may keep its fields in either buffer.
+  auto step = [&](int mode) {
+    const int force = mode == 0;
+    GFIX_PROF(c, PK_CDERIV, hipLaunchKernelGGL(k_cderiv, grid, blk, 0, s, U, G, F, g, sc, n));
     enq_fa<double>(c, F, nullptr, sc.done, sc.map, (int)rows.size());
-    GFIX_PROF(c, PK_CPR, hipLaunchKernelGGL(k_cpr, grid, blk, 0, s, F, F, part, g, sc, cs->nbs));
-    hipLaunchKernelGGL(k_cfin_pr, dim3(T), dim3(1024), 0, s, part, cs->nbs, sc, 0);
-    GFIX_PROF(c, PK_CLINE, hipLaunchKernelGGL(k_cline, grid, blk, 0, s, U, G, F, part, g, sc, cs->nbs, 1));
-    hipLaunchKernelGGL(k_cfin_ls, dim3(T), dim3(1024), 0, s, part, cs->nbs, sc, 1, 0);
-    GFIX_PROF(c, PK_CEXP, hipLaunchKernelGGL(k_cexp, grid, blk, 0, s, G, F, g, sc));
-    GFIX_PROF(c, PK_CUPD, hipLaunchKernelGGL(k_cupdate, grid, blk, 0, s, F, sn, g, sc, 0));
+    GFIX_PROF(c, PK_CPR, hipLaunchKernelGGL(k_cpr, grid, blk, 0, s, F, mode ? O : F, part, g, sc, cs->nbs));
+    if (!fuse) hipLaunchKernelGGL(k_cfin_pr, dim3(T), dim3(1024), 0, s, part, cs->nbs, sc, mode);
+    GFIX_PROF(c, PK_CUPD, hipLaunchKernelGGL(k_cupdate, grid, blk, 0, s, F, sn, g, sc, mode, part, cs->nbs, fuse));
+    GFIX_PROF(c, PK_CLINE, hipLaunchKernelGGL(k_cline, grid, blk, 0, s, U, G, sn, part, g, sc, cs->nbs, force));
+    if (!fuse) hipLaunchKernelGGL(k_cfin_ls, dim3(T), dim3(1024), 0, s, part, cs->nbs, sc, force, 0);
+    GFIX_PROF(c, PK_CEXP, hipLaunchKernelGGL(k_cexp, grid, blk, 0, s, G, sn, g, sc, part, cs->nbs, force, fuse));
     std::swap(F, O);
-  }
+  };
+  if (method == GLU_GFIX_CG) step(0);
   for (;;) {
     for (int b = 0; b < 8; b++) {
-      GFIX_PROF(c, PK_CDERIV, hipLaunchKernelGGL(k_cderiv, grid, blk, 0, s, U, G, F, g, sc));
-      enq_fa<double>(c, F, nullptr, sc.done, sc.map, (int)rows.size());
       if (method == GLU_GFIX_CG) {
-        GFIX_PROF(c, PK_CPR, hipLaunchKernelGGL(k_cpr, grid, blk, 0, s, F, O, part, g, sc, cs->nbs));
-        hipLaunchKernelGGL(k_cfin_pr, dim3(T), dim3(1024), 0, s, part, cs->nbs, sc, 1);
-        GFIX_PROF(c, PK_CUPD, hipLaunchKernelGGL(k_cupdate, grid, blk, 0, s, F, sn, g, sc, 1));
-        GFIX_PROF(c, PK_CLINE, hipLaunchKernelGGL(k_cline, grid, blk, 0, s, U, G, sn, part, g, sc, cs->nbs, 0));
-        hipLaunchKernelGGL(k_cfin_ls, dim3(T), dim3(1024), 0, s, part, cs->nbs, sc, 0, 0);
-        GFIX_PROF(c, PK_CEXP, hipLaunchKernelGGL(k_cexp, grid, blk, 0, s, G, sn, g, sc));
-        std::swap(F, O);
+        step(1);
       } else {
+        GFIX_PROF(c, PK_CDERIV, hipLaunchKernelGGL(k_cderiv, grid, blk, 0, s, U, G, F, g, sc, n));
+        enq_fa<double>(c, F, nullptr, sc.done, sc.map, (int)rows.size());
         hipLaunchKernelGGL(k_cfin_ls, dim3(T), dim3(1024), 0, s, part, cs->nbs, sc, 0, 1);
-        GFIX_PROF(c, PK_CEXP, hipLaunchKernelGGL(k_cexp, grid, blk, 0, s, G, F, g, sc));
+        GFIX_PROF(c, PK_CEXP, hipLaunchKernelGGL(k_cexp, grid, blk, 0, s, G, F, g, sc, part, cs->nbs, 0, 0));
         GFIX_PROF(c, PK_CPR, hipLaunchKernelGGL(k_cpr, grid, blk, 0, s, F, F, part, g, sc, cs->nbs));
         hipLaunchKernelGGL(k_cfin_der, dim3(T), dim3(1024), 0, s, part, cs->nbs, sc);
       }
-      hipLaunchKernelGGL(k_citer_end, dim3(1), dim3(256), 0, s, sc);
+      n++;
     }
+    hipLaunchKernelGGL(k_cstop, dim3(1), dim3(256), 0, s, sc, n);
     if (hipMemcpyAsync(done.data(), sc.done, T * sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
       return gfix_fail(-2, "Coulomb iteration failed: %s", hipGetErrorString(hipGetLastError()));
