@@ -169,6 +169,7 @@ extern "C" int glu_gfix_create(glu_gfix_ctx **out, const size_t dims[4], int gft
   c->precision = precision;
   const long long V = c->g.V;
   c->nblk = (V + kBlock - 1) / kBlock;
+  c->small = small_lattice(c->g);
   int rc = 0;
 #define CK(x)                                                                  \
   do {                                                                         \
@@ -527,15 +528,29 @@ template <typename T> static void swap_cg_buffers(glu_gfix_ctx *c) {
   c->upar[tix<T>()] ^= 1;
   c->fpar[tix<T>()] ^= 1;
 }
-template <typename T> static void enq_update_deriv(glu_gfix_ctx *c) {
+// the theta partials of the update: behind the probe partials, which the
+// small-lattice update reads while it writes them
+static double *theta_part(glu_gfix_ctx *c) { return c->small ? c->part + 12 * c->nblk : c->part; }
+static int part_sub(const glu_gfix_ctx *c) { return c->small ? 4 : 1; }
+// fuse: on a small lattice the update takes its step from the line search's
+// partials (no finaliser has run)
+template <typename T> static void enq_update_deriv(glu_gfix_ctx *c, bool fuse) {
   const Bufs b = bufs_for<T>(c);
   void *nxt = sizeof(T) == 4 ? c->U32b : c->U64b;
   GFIX_PROF(c, pk<T>(PK_EGDERIV),
-            launch_egauge_deriv<T>(b.U, nxt, b.sn, b.G, b.F, b.old, c->part, geo_order(c, c->ord_eg), c->ctrl,
-                                   c->stream));
+            c->small ? launch_egauge_deriv_small<T>(b.U, nxt, b.sn, b.G, b.old, theta_part(c), c->g, c->ctrl, c->part,
+                                                    fuse ? c->nblk : 0, c->stream)
+                     : launch_egauge_deriv<T>(b.U, nxt, b.sn, b.G, b.F, b.old, c->part, geo_order(c, c->ord_eg),
+                                              c->ctrl, c->stream));
   swap_cg_buffers<T>(c);
   c->deriv_ready[tix<T>()] = 1;
   c->run.nenq++;
+}
+template <typename T> static void enq_line_search(glu_gfix_ctx *c, const void *U, const void *D, int force) {
+  if (c->small)
+    launch_line_search_small<T>(U, D, c->part, c->g, c->ctrl, force, c->stream);
+  else
+    launch_line_search<T>(U, D, c->part, geo_order(c, c->ord_ls), c->ctrl, force, c->stream);
 }
 
 // SD start of steep_Landau_FACG, Gfix/FACG.c:249-265.  sn = in_old = in and
@@ -548,18 +563,20 @@ template <typename T> static void enq_sd_start(glu_gfix_ctx *c, const Bufs &b) {
   launch_deriv<T>(b.U, b.F, c->part, geo_order(c, c->ord_eg), c->ctrl, s);
   launch_fin_theta(c->part, c->nblk, c->ctrl, landau_norm(c), s);
   enq_fa<T>(c, b.F, c->ctrl, nullptr);
-  launch_line_search<T>(b.U, b.F, c->part, geo_order(c, c->ord_ls), c->ctrl, 1, s);
-  launch_fin_ls(c->part, c->nblk, c->ctrl, c->trace, 1, 0.15, 0.30, s);
+  enq_line_search<T>(c, b.U, b.F, 1);
+  launch_fin_ls(c->part, c->nblk, c->ctrl, c->trace, 1, 0.15, 0.30, s, part_sub(c));
   launch_copy<T>(b.F, b.sn, c->g.V, c->ctrl, s);
   launch_pr_sums<T>(b.F, b.F, c->part, c->g.V, c->ctrl, s);
   launch_fin_sd(c->part, c->nblk, c->ctrl, s);
-  enq_update_deriv<T>(c);
-  launch_fin_theta(c->part, c->nblk, c->ctrl, landau_norm(c), s);
+  enq_update_deriv<T>(c, false);
+  launch_fin_theta(theta_part(c), c->nblk, c->ctrl, landau_norm(c), s, part_sub(c));
 }
 
 // one FACG iteration (Gfix/FACG.c:272-334).  On entry with a pending
 // derivative, theta of the current links is already in the control block
-// (set with the end of the previous iteration or the SD start).
+// (set with the end of the previous iteration or the SD start).  On a small
+// lattice the direction update and the gauge update take beta and the step
+// from the partial sums themselves.
 template <typename T> static void enq_cg_iter(glu_gfix_ctx *c, const Bufs &b) {
   hipStream_t s = c->stream;
   if (!c->deriv_ready[tix<T>()]) {
@@ -569,13 +586,13 @@ template <typename T> static void enq_cg_iter(glu_gfix_ctx *c, const Bufs &b) {
   }
   enq_fa<T>(c, b.F, c->ctrl, nullptr);
   GFIX_PROF(c, pk<T>(PK_PR), launch_pr_sums<T>(b.F, b.old, c->part, c->g.V, c->ctrl, s));
-  launch_fin_pr(c->part, c->nblk, c->ctrl, s);
-  GFIX_PROF(c, pk<T>(PK_CGUPD), launch_cg_update<T>(b.F, b.sn, c->g.V, c->ctrl, s));
-  GFIX_PROF(c, pk<T>(PK_LSEARCH),
-            launch_line_search<T>(b.U, b.sn, c->part, geo_order(c, c->ord_ls), c->ctrl, 0, s));
-  launch_fin_ls(c->part, c->nblk, c->ctrl, c->trace, 0, 0.15, 0.30, s);
-  enq_update_deriv<T>(c);
-  launch_fin_iter(c->part, c->nblk, c->ctrl, c->trace, landau_norm(c), s);
+  if (!c->small) launch_fin_pr(c->part, c->nblk, c->ctrl, s);
+  GFIX_PROF(c, pk<T>(PK_CGUPD),
+            launch_cg_update<T>(b.F, b.sn, c->g.V, c->ctrl, s, c->part, c->small ? c->nblk : 0));
+  GFIX_PROF(c, pk<T>(PK_LSEARCH), enq_line_search<T>(c, b.U, b.sn, 0));
+  if (!c->small) launch_fin_ls(c->part, c->nblk, c->ctrl, c->trace, 0, 0.15, 0.30, s);
+  enq_update_deriv<T>(c, true);
+  launch_fin_iter(theta_part(c), c->nblk, c->ctrl, c->trace, landau_norm(c), s, part_sub(c));
 }
 
 // one FASD iteration (Gfix/FACG.c:202-235, fixed step GF_TUNE)

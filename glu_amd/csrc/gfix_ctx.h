@@ -97,6 +97,7 @@ struct glu_gfix_ctx {
   void *F = nullptr, *sn = nullptr, *old = nullptr;
   double *part = nullptr;  // per-block partial sums
   long long nblk = 0;
+  int small = 0;  // the iteration runs the small-lattice kernels
   gfix::Ctrl *ctrl = nullptr;   // device control block
   gfix::Ctrl *hctrl = nullptr;  // pinned host mirror
   double *trace = nullptr;

@@ -153,6 +153,41 @@ template <typename T> struct DerivAcc {
   }
 };
 
+// one direction's terms of DerivAcc::add, and the sum of four directions'
+// terms in its order: add(q, s) for mu = 0..3
+template <typename T> struct DerivTerms {
+  T v[10];
+  __device__ __forceinline__ DerivTerms(const su3<T> &q, const su3<T> &s) {
+    v[0] = T(2) * s.e[0].im - s.e[4].im - s.e[8].im;
+    v[1] = T(-2) * q.e[0].im + q.e[4].im + q.e[8].im;
+    v[2] = s.e[1].re - s.e[3].re - q.e[1].re + q.e[3].re;
+    v[3] = s.e[1].im + s.e[3].im - q.e[1].im - q.e[3].im;
+    v[4] = s.e[2].re - s.e[6].re - q.e[2].re + q.e[6].re;
+    v[5] = s.e[2].im + s.e[6].im - q.e[2].im - q.e[6].im;
+    v[6] = T(2) * s.e[4].im - s.e[0].im - s.e[8].im;
+    v[7] = T(-2) * q.e[4].im + q.e[0].im + q.e[8].im;
+    v[8] = s.e[5].re - s.e[7].re - q.e[5].re + q.e[7].re;
+    v[9] = s.e[5].im + s.e[7].im - q.e[5].im - q.e[7].im;
+  }
+};
+template <typename T, typename Term> __device__ __forceinline__ DerivAcc<T> deriv_sum(Term term) {
+  DerivAcc<T> d;
+#pragma unroll
+  for (int mu = 0; mu < 4; mu++) {
+    d.R0 += term(mu, 0);
+    d.R0 += term(mu, 1);
+    d.R1 += term(mu, 2);
+    d.I1 += term(mu, 3);
+    d.R2 += term(mu, 4);
+    d.I2 += term(mu, 5);
+    d.R3 += term(mu, 6);
+    d.R3 += term(mu, 7);
+    d.R4 += term(mu, 8);
+    d.I4 += term(mu, 9);
+  }
+  return d;
+}
+
 // parabola vertex through the three probes, clamped: Gfix/line_search.c:38-57
 __device__ __forceinline__ double approx_minimum(const double al[3], const double f[3]) {
   const double A = f[0] / ((al[0] - al[1]) * (al[0] - al[2]));

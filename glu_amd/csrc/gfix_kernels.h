@@ -61,12 +61,22 @@ void launch_deriv(const void *U, void *F, double *part, const Geo &g, const Ctrl
 template <typename T>
 void launch_pr_sums(const void *F, const void *O, double *part, long long V, const Ctrl *ctrl, hipStream_t s);
 template <typename T>
-void launch_cg_update(const void *F, void *sn, long long V, const Ctrl *ctrl, hipStream_t s);
+void launch_cg_update(const void *F, void *sn, long long V, Ctrl *ctrl, hipStream_t s, const double *part = nullptr,
+                      long long nb = 0);
 template <typename T>
 void launch_copy(const void *F, void *a, long long V, const Ctrl *ctrl, hipStream_t s);
 template <typename T>
 void launch_line_search(const void *U, const void *F, double *part, const Geo &g, const Ctrl *ctrl, int force,
                         hipStream_t s);
+// small lattices: four workgroups of 64 sites in the place of each of 256,
+// whose partial sums stay separate (12 and 4 numbers a row of nblk)
+bool small_lattice(const Geo &g);
+template <typename T>
+void launch_line_search_small(const void *U, const void *F, double *part, const Geo &g, const Ctrl *ctrl, int force,
+                              hipStream_t s);
+template <typename T>
+void launch_egauge_deriv_small(const void *Uin, void *Uout, const void *D, void *G, void *Fout, double *part,
+                               const Geo &g, Ctrl *ctrl, const double *probe, long long nb, hipStream_t s);
 template <typename T>
 void launch_egauge(void *U, const void *F, void *G, const Geo &g, const Ctrl *ctrl, int fixed, hipStream_t s);
 template <typename T>
@@ -76,14 +86,15 @@ void launch_pack(const double *aos, void *U, long long V, long long site0, long 
 void launch_unpack(const void *U, double *aos, long long V, long long site0, long long n, hipStream_t s);
 template <typename T> void launch_identity(void *G, long long V, hipStream_t s);
 
-void launch_fin_theta(const double *part, long long nb, Ctrl *ctrl, double norm, hipStream_t s);
+void launch_fin_theta(const double *part, long long nb, Ctrl *ctrl, double norm, hipStream_t s, int sub = 1);
 void launch_fin_pr(const double *part, long long nb, Ctrl *ctrl, hipStream_t s);
 void launch_fin_sd(const double *part, long long nb, Ctrl *ctrl, hipStream_t s);
 void launch_fin_ls(const double *part, long long nb, Ctrl *ctrl, double *trace, int force, double pl1, double pl2,
-                   hipStream_t s);
+                   hipStream_t s, int sub = 1);
 void launch_iter_end(Ctrl *ctrl, double *trace, int fasd, hipStream_t s);
 void launch_sum_part(const double *part, long long nb, double *out, hipStream_t s);
-void launch_fin_iter(const double *part, long long nb, Ctrl *ctrl, double *trace, double norm, hipStream_t s);
+void launch_fin_iter(const double *part, long long nb, Ctrl *ctrl, double *trace, double norm, hipStream_t s,
+                     int sub = 1);
 void launch_begin_segment(Ctrl *ctrl, int sd, hipStream_t s);
 void launch_demote(const void *U, void *W, long long n, hipStream_t s);
 void launch_apply_gauge(void *U, const void *G, const Geo &g, hipStream_t s);

@@ -65,14 +65,79 @@ __global__ __launch_bounds__(kBlock) void k_pr_sums(const vec2<T> *__restrict__ 
   block_sum_store<2>(v, part + 2 * blockIdx.x);
 }
 
+// Small lattices (up to kSmallBlocks partial rows) run without the
+// single-block finalisers of the PR sums and of the line search: every block
+// of the kernel that needs beta or the step adds the partial rows itself, in
+// the order of final_sum, and block 0 writes the scalars, none of which the
+// kernel's other blocks read.  At 8^4 a finaliser took 3 to 4 us of an
+// iteration's 47.  The line: one row for each thread of a block.  Iteration
+// with and without the small-lattice kernels (FP64 / mixed, us): 4^4 41 / 41
+// and 52 / 52, 8^4 34 / 42 and 47 / 56, 12^4 58 / 63 and 69 / 76, 14^4 73 /
+// 78 and 81 / 89, 16^4 71 / 70 and 72 / 73: at 16^4 every CU has its
+// wavefronts without the split and the gain ends.
+constexpr long long kSmallBlocks = 256;
+// one row a thread; a row may be kept as the 4 sums of its block's waves
+template <int NV>
+__device__ __forceinline__ void small_sum(const double *__restrict__ part, long long nb, int sub, double (&out)[NV]) {
+  __shared__ double sh[NV][kBlock / kWave];
+  const int b = threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < NV; k++) {
+    double v = 0.0;
+    if (b < nb) {
+      if (sub == 1)
+        v = part[(long long)b * NV + k];
+      else
+        for (int j = 0; j < 4; j++) v += part[((long long)b * 4 + j) * NV + k];
+    }
+    v = wave_sum(v);
+    if (threadIdx.x % kWave == 0) sh[k][threadIdx.x / kWave] = v;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NV; k++) {
+    out[k] = 0.0;
+    for (int j = 0; j < kBlock / kWave; j++) out[k] += sh[k][j];
+  }
+}
+
+// beta: Polak-Ribiere clipped at 0, Fletcher-Reeves below CG_TOL
+// (Gfix/FACG.c:306-313)
+__device__ __forceinline__ double pr_beta(const Ctrl *ctrl, double insum, double sc) {
+  double beta = sc / ctrl->inold;
+  if (beta < 0.0) beta = 0.0;
+  if (ctrl->theta < ctrl->cg_tol) beta = insum / ctrl->inold;
+  if (ctrl->switch_theta > 0.0) {  // safeguards of the mixed FP32 phase
+    if ((ctrl->sg_mode & 1) && ctrl->sg_uphill) beta = 0.0;
+    if ((ctrl->sg_mode & 2) && beta > ctrl->beta_cap) beta = ctrl->beta_cap;
+  }
+  return beta;
+}
+__device__ __forceinline__ void pr_record(Ctrl *ctrl, double insum, double sc, double beta) {
+  ctrl->insum = insum;  // becomes inold with the step (ls_record)
+  ctrl->sum_conj = sc;
+  ctrl->beta = beta;
+}
+
 // sn = in + beta sn (Gfix/FACG.c:315-323).  GLU's old = in needs no copy:
 // the fused update writes the next derivative into the field buffer that
 // held in_old, and the host swaps the two, so `in` becomes in_old in place.
+// nb > 0: beta comes from the nb partial rows of the PR sums.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_cg_update(const vec2<T> *__restrict__ F, vec2<T> *__restrict__ sn,
-                                                     long long n4, const Ctrl *__restrict__ ctrl) {
+                                                     long long n4, Ctrl *ctrl, const double *__restrict__ part,
+                                                     long long nb) {
   if (ctrl->done) return;
-  const T beta = (T)ctrl->beta;
+  double b;
+  if (nb > 0) {
+    double s[2];
+    small_sum<2>(part, nb, 1, s);
+    b = pr_beta(ctrl, s[0], s[1]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) pr_record(ctrl, s[0], s[1], b);
+  } else {
+    b = ctrl->beta;
+  }
+  const T beta = (T)b;
   for (long long j = (long long)blockIdx.x * blockDim.x + threadIdx.x; j < n4; j += (long long)gridDim.x * blockDim.x) {
     const cx<T> a = ld<T>(F + j), b = ld<T>(sn + j);
     st<T>(sn + j, mk<T>(a.re + beta * b.re, a.im + beta * b.im));
@@ -147,13 +212,13 @@ __device__ __forceinline__ void probe_cols(const cx<double> (&f)[4], cx<double> 
     c[pr][3] = m.e[1], c[pr][4] = m.e[4], c[pr][5] = m.e[7];
   }
 }
-// site of this thread: in FP32 a workgroup owns an 8 x 4 x 4 x 2 tile
-__device__ __forceinline__ long long probe_site(const Geo &g, unsigned lb, double) {
-  return (long long)lb * blockDim.x + threadIdx.x;
+// site of thread t of block lb: in FP32 a block owns an 8 x 4 x 4 x 2 tile
+__device__ __forceinline__ long long probe_site(const Geo &g, unsigned lb, unsigned t, double) {
+  return (long long)lb * kBlock + t;
 }
-__device__ __forceinline__ long long probe_site(const Geo &g, unsigned lb, float) {
+__device__ __forceinline__ long long probe_site(const Geo &g, unsigned lb, unsigned t, float) {
   const unsigned nx = (unsigned)g.L[0] / 8, ny = (unsigned)g.L[1] / 4, nz = (unsigned)g.L[2] / 4;
-  const unsigned t = threadIdx.x, by = lb / nx, bz = by / ny, bt = bz / nz;
+  const unsigned by = lb / nx, bz = by / ny, bt = bz / nz;
   const long long x = (lb - by * nx) * 8 + (t & 7u), y = (by - bz * ny) * 4 + (t >> 3 & 3u);
   const long long z = (bz - bt * nz) * 4 + (t >> 5 & 3u), tt = bt * 2 + (t >> 7);
   return x + g.S[1] * y + g.S[2] * z + g.S[3] * tt;
@@ -167,7 +232,7 @@ __global__ __launch_bounds__(kBlock) void k_line_search(const vec2<T> *__restric
   if (!force && !(ctrl->theta > ctrl->cg_tol)) return;
   const long long V = g.V;
   const unsigned lb = logical_block(g);
-  const long long i = probe_site(g, lb, T(0));
+  const long long i = probe_site(g, lb, threadIdx.x, T(0));
   double v[3] = {0.0, 0.0, 0.0};
   if (i < V) {
     int x[4];
@@ -244,6 +309,80 @@ __global__ __launch_bounds__(kBlock) void k_line_search_rows(const float2 *__res
   block_sum_store<3>(v, part + 3 * lb);
 }
 
+// The probes of a small lattice: one wave per direction of 64 sites, so that
+// a lattice of fewer sites than the GPU has lanes runs four times the waves,
+// each a quarter of the chain.  The sites of a block of k_line_search (or
+// k_line_search_rows) are four workgroups here, whose three sums stay
+// separate in part; the terms and the order of their addition are the same.
+// 8^4: 4.3 us, 9.0 with one thread per site.
+enum { PROBE_COLS = 0, PROBE_ROWS = 1 };
+template <typename T, int KIND>
+__global__ __launch_bounds__(kBlock) void k_line_search_small(const vec2<T> *__restrict__ U,
+                                                             const vec2<T> *__restrict__ F, double *__restrict__ part,
+                                                             Geo g, const Ctrl *__restrict__ ctrl, int force) {
+  if (ctrl->done) return;
+  if (!force && !(ctrl->theta > ctrl->cg_tol)) return;
+  __shared__ double sh[3][4][kWave];
+  const long long V = g.V;
+  const unsigned lb = blockIdx.x >> 2, w = blockIdx.x & 3u;
+  const int lane = threadIdx.x % kWave, mu = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const long long i = KIND == PROBE_ROWS ? (long long)lb * kBlock + w * kWave + lane
+                                         : probe_site(g, lb, w * kWave + lane, T(0));
+  double v[3] = {0.0, 0.0, 0.0};
+  if (i < V) {
+    int x[4];
+    coords(g, i, x);
+    if constexpr (KIND == PROBE_ROWS) {
+      // the loops of k_line_search_rows, one direction long: which product
+      // of a sum is fused depends on what shares a basic block with it, and
+      // the FP32 schedule keeps that kernel's rounding
+      int end = mu + 1;
+      asm("" : "+s"(end));
+#pragma unroll 1
+      for (int pr = 1; pr <= 2; pr++) {
+        const double al = pr == 1 ? 0.15 : 0.30;
+        const su3<double> A = gauge_at64<T>(F, V, i, al);
+        double acc = 0.0;
+#pragma unroll 1
+        for (int d = mu; d < end; d++) {
+          cx<double> au[6];
+          {
+            const su3<double> u = promote(load_link<float>(U, d, i, V));
+            if (pr == 1) v[0] += u.e[0].re + u.e[4].re + u.e[8].re;
+            ab_rows01<double>(A, u, au);
+          }
+          acc += retrace_rows01_dag<double>(au, gauge_at64<T>(F, V, nb_fwd(g, i, x, d), al));
+        }
+        v[pr] = acc;
+      }
+    } else {
+      cx<double> f[4], u[6], A[2][6], B[2][6];
+      field_at<T>(F, V, i, f);
+      probe_cols(f, A, T(0));
+      load_cols<T>(U, mu, i, V, u);
+      field_at<T>(F, V, nb_fwd(g, i, x, mu), f);
+      v[0] = u[0].re + u[4].re + (u[0].re * u[4].re - u[0].im * u[4].im) - (u[1].re * u[3].re - u[1].im * u[3].im);
+      probe_cols(f, B, T(0));
+#pragma unroll
+      for (int pr = 0; pr < 2; pr++) {
+        cx<double> a2[3], M[6];
+        third_col(A[pr], a2);
+        mul_cols01(A[pr], a2, u, M);
+        v[1 + pr] = retrace_cols(M, B[pr]);
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 3; k++) sh[k][mu][lane] = v[k];
+  __syncthreads();
+  if (mu < 3) {  // wave k adds sum k: the directions in order, then the sites
+    double s = 0.0;
+    for (int d = 0; d < 4; d++) s += sh[mu][d][lane];
+    s = wave_sum(s);
+    if (lane == 0) part[3 * (long long)blockIdx.x + mu] = s;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // U_mu(x) <- g(x) U_mu(x) g(x+mu)^dagger: Gfix/line_search.c:60-97.
 // With G != null the site transform is also accumulated in FP64,
@@ -277,6 +416,42 @@ __global__ __launch_bounds__(kBlock) void k_egauge(vec2<T> *__restrict__ U, cons
     const su3<double> A64 = gauge_at64<T>(F, V, i, alpha);
     store_link<double>(G, 0, i, V, mul_cols<double>(A64, load_link<double>(G, 0, i, V)));
   }
+}
+
+// the step of an iteration from its probe sums: parabola vertex
+// (Gfix/line_search.c:274-341), or GF_TUNE below CG_TOL
+__device__ __forceinline__ bool ls_runs(const Ctrl *ctrl, int force) { return force || (ctrl->theta > ctrl->cg_tol); }
+struct LsStep {
+  double alpha, probe[3];
+  int uphill;
+};
+__device__ __forceinline__ LsStep ls_step(const Ctrl *ctrl, const double (&s)[3], bool do_ls, int force, double pl1,
+                                          double pl2) {
+  LsStep r{ctrl->gf_alpha, {0.0, 0.0, 0.0}, 0};
+  if (!do_ls) return r;
+  double val[3];
+  for (int k = 0; k < 3; k++) {
+    const double tot = s[k] + (ctrl->sd_start ? ctrl->stale_probe[k] : 0.0);
+    r.probe[k] = tot;
+    val[k] = -tot;
+  }
+  const double al[3] = {0.0, pl1, pl2};
+  r.alpha = approx_minimum(al, val);
+  // mixed FP32 phase: the functional rises along the direction
+  const int sg = ctrl->switch_theta > 0.0 && !force ? ctrl->sg_mode : 0;
+  r.uphill = sg && val[1] > val[0];
+  if ((sg & 4) && r.uphill) r.alpha = 0.0;
+  return r;
+}
+__device__ __forceinline__ void ls_record(Ctrl *ctrl, const LsStep &r, bool do_ls, int force) {
+  ctrl->upd++;  // the gauge update that follows will run
+  if (do_ls)
+    for (int k = 0; k < 3; k++) ctrl->probe[k] = r.probe[k];
+  ctrl->alpha = r.alpha;
+  ctrl->did_ls = do_ls;
+  if (force) return;
+  ctrl->sg_uphill = r.uphill;
+  ctrl->inold = ctrl->insum;  // beta has been taken
 }
 
 // ---------------------------------------------------------------------------
@@ -331,18 +506,84 @@ __global__ __launch_bounds__(kBlock) void k_egauge_deriv(const vec2<T> *__restri
   block_sum_store<1>(loc, part + lb);
 }
 
+// k_egauge_deriv on a small lattice: one wave per direction of 64 sites (see
+// k_line_search_small), each thread one link, its backward link and their
+// terms of the divergence, which wave 0 adds in the order of DerivAcc.  nb >
+// 0: the step comes from the probe partials probe[12 nb] of the line search.
+// 8^4: 7.4 us, 12 with one thread per site.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_egauge_deriv_small(const vec2<T> *__restrict__ Uin,
+                                                              vec2<T> *__restrict__ Uout,
+                                                              const vec2<T> *__restrict__ D, double2 *__restrict__ G,
+                                                              vec2<T> *__restrict__ Fout, double *__restrict__ part,
+                                                              Geo g, Ctrl *ctrl, const double *__restrict__ probe,
+                                                              long long nb) {
+  if (ctrl->done) return;
+  __shared__ T sh[10][4][kWave];
+  double alpha;
+  if (nb > 0) {
+    const bool do_ls = ls_runs(ctrl, 0);
+    double s[3] = {0.0, 0.0, 0.0};
+    if (do_ls) small_sum<3>(probe, nb, 4, s);
+    const LsStep r = ls_step(ctrl, s, do_ls, 0, 0.15, 0.30);
+    alpha = r.alpha;
+    if (blockIdx.x == 0 && threadIdx.x == 0) ls_record(ctrl, r, do_ls, 0);
+  } else {
+    alpha = ctrl->alpha;
+  }
+  const long long V = g.V;
+  const int lane = threadIdx.x % kWave, mu = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const long long i = (long long)blockIdx.x * kWave + lane;
+  if (i < V) {
+    int x[4];
+    coords(g, i, x);
+    const su3<T> A = gauge_at<T>(D, V, i, (T)alpha);
+    const su3<T> B = gauge_at<T>(D, V, nb_fwd(g, i, x, mu), (T)alpha);
+    su3<T> n = gtransform<T>(A, load_link<T>(Uin, mu, i, V), B);
+    if (sizeof(T) == 4) gram_reunit<T>(n);
+    store_link<T>(Uout, mu, i, V, n);
+    const long long xb = nb_bwd(g, i, x, mu);
+    const su3<T> C = gauge_at<T>(D, V, xb, (T)alpha);
+    su3<T> sb = gtransform<T>(C, load_link<T>(Uin, mu, xb, V), A);
+    if (sizeof(T) == 4) gram_reunit<T>(sb);
+    const DerivTerms<T> t(n, sb);
+#pragma unroll
+    for (int k = 0; k < 10; k++) sh[k][mu][lane] = t.v[k];
+    if (G && mu == 3) {
+      const su3<double> A64 = gauge_at64<T>(D, V, i, alpha);
+      store_link<double>(G, 0, i, V, mul_cols<double>(A64, load_link<double>(G, 0, i, V)));
+    }
+  }
+  __syncthreads();
+  if (mu == 0) {
+    double s = 0.0;
+    if (i < V) s = deriv_sum<T>([&](int m, int k) { return sh[k][m][lane]; }).store(Fout, V, i);
+    s = wave_sum(s);
+    if (lane == 0) part[blockIdx.x] = s;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // single-block finalisers (fixed summation order)
 // ---------------------------------------------------------------------------
+// sub = 4: a row is kept as the 4 sums of its block's waves
 template <int NV>
-__device__ __forceinline__ void final_sum(const double *__restrict__ part, long long nb, double (&out)[NV]) {
+__device__ __forceinline__ void final_sum(const double *__restrict__ part, long long nb, double (&out)[NV],
+                                          int sub = 1) {
   __shared__ double sh[NV][1024 / kWave];
   double v[NV];
 #pragma unroll
   for (int k = 0; k < NV; k++) v[k] = 0.0;
   for (long long b = threadIdx.x; b < nb; b += blockDim.x)
 #pragma unroll
-    for (int k = 0; k < NV; k++) v[k] += part[b * NV + k];
+    for (int k = 0; k < NV; k++) {
+      double r = 0.0;
+      if (sub == 1)
+        r = part[b * NV + k];
+      else
+        for (int j = 0; j < 4; j++) r += part[(b * 4 + j) * NV + k];
+      v[k] += r;
+    }
   const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
 #pragma unroll
   for (int k = 0; k < NV; k++) {
@@ -359,10 +600,10 @@ __device__ __forceinline__ void final_sum(const double *__restrict__ part, long 
 }
 
 // theta = sum / (NC V): GFNORM_LANDAU, Headers/GLU_definitions.h:427
-__global__ void k_fin_theta(const double *__restrict__ part, long long nb, Ctrl *ctrl, double norm) {
+__global__ void k_fin_theta(const double *__restrict__ part, long long nb, Ctrl *ctrl, double norm, int sub) {
   if (ctrl->done) return;
   double s[1];
-  final_sum<1>(part, nb, s);
+  final_sum<1>(part, nb, s, sub);
   if (threadIdx.x == 0) {
     double th = s[0] * norm;
     if (ctrl->sd_start) th += ctrl->stale_theta;  // GLU's stale red[5] slots
@@ -370,27 +611,11 @@ __global__ void k_fin_theta(const double *__restrict__ part, long long nb, Ctrl 
   }
 }
 
-// beta: Polak-Ribiere clipped at 0, Fletcher-Reeves below CG_TOL
-// (Gfix/FACG.c:306-313)
 __global__ void k_fin_pr(const double *__restrict__ part, long long nb, Ctrl *ctrl) {
   if (ctrl->done) return;
   double s[2];
   final_sum<2>(part, nb, s);
-  if (threadIdx.x == 0) {
-    const double insum = s[0], sc = s[1];
-    double beta = sc / ctrl->inold;
-    if (beta < 0.0) beta = 0.0;
-    if (ctrl->theta < ctrl->cg_tol) beta = insum / ctrl->inold;
-    if (ctrl->switch_theta > 0.0) {  // safeguards of the mixed FP32 phase
-      if ((ctrl->sg_mode & 1) && ctrl->sg_uphill) beta = 0.0;
-      if ((ctrl->sg_mode & 2) && beta > ctrl->beta_cap) beta = ctrl->beta_cap;
-    }
-    ctrl->sg_uphill = 0;
-    ctrl->inold = insum;
-    ctrl->insum = insum;
-    ctrl->sum_conj = sc;
-    ctrl->beta = beta;
-  }
+  if (threadIdx.x == 0) pr_record(ctrl, s[0], s[1], pr_beta(ctrl, s[0], s[1]));
 }
 
 // end of the SD start: inold = sum_DER3 (+ GLU's stale red[3] slots)
@@ -410,31 +635,13 @@ __global__ void k_fin_sd(const double *__restrict__ part, long long nb, Ctrl *ct
 }
 
 __global__ void k_fin_ls(const double *__restrict__ part, long long nb, Ctrl *ctrl, double *trace, int force,
-                         double pl1, double pl2) {
+                         double pl1, double pl2, int sub) {
   if (ctrl->done) return;
-  const int do_ls = force || (ctrl->theta > ctrl->cg_tol);
+  const bool do_ls = ls_runs(ctrl, force);
   double s[3] = {0.0, 0.0, 0.0};
-  if (do_ls) final_sum<3>(part, nb, s);
+  if (do_ls) final_sum<3>(part, nb, s, sub);
   if (threadIdx.x == 0) {
-    ctrl->upd++;  // the gauge update enqueued after this launch will run
-    if (do_ls) {
-      double val[3];
-      for (int k = 0; k < 3; k++) {
-        const double tot = s[k] + (ctrl->sd_start ? ctrl->stale_probe[k] : 0.0);
-        ctrl->probe[k] = tot;
-        val[k] = -tot;
-      }
-      const double al[3] = {0.0, pl1, pl2};
-      ctrl->alpha = approx_minimum(al, val);
-      ctrl->did_ls = 1;
-      // mixed FP32 phase: the functional rises along the direction
-      const int sg = ctrl->switch_theta > 0.0 && !force ? ctrl->sg_mode : 0;
-      ctrl->sg_uphill = sg && val[1] > val[0];
-      if ((sg & 4) && ctrl->sg_uphill) ctrl->alpha = 0.0;
-    } else {
-      ctrl->alpha = ctrl->gf_alpha;
-      ctrl->did_ls = 0;
-    }
+    ls_record(ctrl, ls_step(ctrl, s, do_ls, force, pl1, pl2), do_ls, force);
     if (ctrl->sd_start && trace && ctrl->trace_n < ctrl->trace_cap) {
       double *r = trace + 3 * ctrl->trace_n;
       r[0] = ctrl->theta;
@@ -489,10 +696,11 @@ __global__ void k_iter_end(Ctrl *ctrl, double *trace, int fasd) {
 // partials of the fused update + derivative (as k_fin_theta; the SD start
 // is over, so no stale slots enter).  A stopped run keeps the theta it
 // tested, and the derivative it left is taken again if a segment resumes.
-__global__ void k_fin_iter(const double *__restrict__ part, long long nb, Ctrl *ctrl, double *trace, double norm) {
+__global__ void k_fin_iter(const double *__restrict__ part, long long nb, Ctrl *ctrl, double *trace, double norm,
+                           int sub) {
   if (ctrl->done) return;
   double s[1];
-  final_sum<1>(part, nb, s);
+  final_sum<1>(part, nb, s, sub);
   if (threadIdx.x == 0 && !iter_end_body(ctrl, trace, 0)) ctrl->theta = s[0] * norm;
 }
 
@@ -725,22 +933,26 @@ void launch_pr_sums(const void *F, const void *O, double *part, long long V, con
                      V, ctrl);
 }
 template <typename T>
-void launch_cg_update(const void *F, void *sn, long long V, const Ctrl *ctrl, hipStream_t s) {
+void launch_cg_update(const void *F, void *sn, long long V, Ctrl *ctrl, hipStream_t s, const double *part,
+                      long long nb) {
   const long long n4 = 4 * V;
   const unsigned b = (unsigned)std::min<long long>(nblk(n4), 8192);
-  hipLaunchKernelGGL(k_cg_update<T>, dim3(b), dim3(kBlock), 0, s, (const vec2<T> *)F, (vec2<T> *)sn, n4, ctrl);
+  hipLaunchKernelGGL(k_cg_update<T>, dim3(b), dim3(kBlock), 0, s, (const vec2<T> *)F, (vec2<T> *)sn, n4, ctrl, part,
+                     nb);
 }
 template <typename T> void launch_copy(const void *F, void *a, long long V, const Ctrl *ctrl, hipStream_t s) {
   const long long n4 = 4 * V;
   const unsigned b = (unsigned)std::min<long long>(nblk(n4), 8192);
   hipLaunchKernelGGL(k_copy<T>, dim3(b), dim3(kBlock), 0, s, (const vec2<T> *)F, (vec2<T> *)a, n4, ctrl);
 }
+// whether the FP32 line search's tiles divide the lattice
+static bool probe_tiles(const Geo &g) { return !(g.L[0] % 8 || g.L[1] % 4 || g.L[2] % 4 || g.L[3] % 2); }
 template <typename T>
 void launch_line_search(const void *U, const void *F, double *part, const Geo &g, const Ctrl *ctrl, int force,
                         hipStream_t s) {
   if constexpr (sizeof(T) == 4) {
     Geo gt = g;
-    if (g.L[0] % 8 || g.L[1] % 4 || g.L[2] % 4 || g.L[3] % 2) {
+    if (!probe_tiles(g)) {
       hipLaunchKernelGGL(k_line_search_rows, dim3(nblk(g.V)), dim3(kBlock), 0, s, (const float2 *)U,
                          (const float2 *)F, part, g, ctrl, force);
       return;
@@ -752,6 +964,27 @@ void launch_line_search(const void *U, const void *F, double *part, const Geo &g
     hipLaunchKernelGGL(k_line_search<T>, dim3(nblk(g.V)), dim3(kBlock), 0, s, (const vec2<T> *)U,
                        (const vec2<T> *)F, part, g, ctrl, force);
   }
+}
+bool small_lattice(const Geo &g) { return nblk(g.V) <= kSmallBlocks; }
+template <typename T>
+void launch_line_search_small(const void *U, const void *F, double *part, const Geo &g, const Ctrl *ctrl, int force,
+                              hipStream_t s) {
+  const dim3 grid(4 * nblk(g.V)), blk(kBlock);
+  if constexpr (sizeof(T) == 4) {
+    if (!probe_tiles(g)) {
+      hipLaunchKernelGGL((k_line_search_small<T, PROBE_ROWS>), grid, blk, 0, s, (const vec2<T> *)U,
+                         (const vec2<T> *)F, part, g, ctrl, force);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_line_search_small<T, PROBE_COLS>), grid, blk, 0, s, (const vec2<T> *)U, (const vec2<T> *)F,
+                     part, g, ctrl, force);
+}
+template <typename T>
+void launch_egauge_deriv_small(const void *Uin, void *Uout, const void *D, void *G, void *Fout, double *part,
+                               const Geo &g, Ctrl *ctrl, const double *probe, long long nb, hipStream_t s) {
+  hipLaunchKernelGGL(k_egauge_deriv_small<T>, dim3(4 * nblk(g.V)), dim3(kBlock), 0, s, (const vec2<T> *)Uin,
+                     (vec2<T> *)Uout, (const vec2<T> *)D, (double2 *)G, (vec2<T> *)Fout, part, g, ctrl, probe, nb);
 }
 template <typename T>
 void launch_egauge(void *U, const void *F, void *G, const Geo &g, const Ctrl *ctrl, int fixed, hipStream_t s) {
@@ -771,7 +1004,12 @@ template <typename T> void launch_identity(void *G, long long V, hipStream_t s) 
 #define GFIX_INST(T)                                                                                          \
   template void launch_deriv<T>(const void *, void *, double *, const Geo &, const Ctrl *, hipStream_t);      \
   template void launch_pr_sums<T>(const void *, const void *, double *, long long, const Ctrl *, hipStream_t); \
-  template void launch_cg_update<T>(const void *, void *, long long, const Ctrl *, hipStream_t);               \
+  template void launch_cg_update<T>(const void *, void *, long long, Ctrl *, hipStream_t, const double *,      \
+                                    long long);                                                               \
+  template void launch_line_search_small<T>(const void *, const void *, double *, const Geo &, const Ctrl *,  \
+                                            int, hipStream_t);                                                \
+  template void launch_egauge_deriv_small<T>(const void *, void *, const void *, void *, void *, double *,    \
+                                             const Geo &, Ctrl *, const double *, long long, hipStream_t);    \
   template void launch_copy<T>(const void *, void *, long long, const Ctrl *, hipStream_t);                    \
   template void launch_line_search<T>(const void *, const void *, double *, const Geo &, const Ctrl *, int,   \
                                       hipStream_t);                                                           \
@@ -782,8 +1020,8 @@ template <typename T> void launch_identity(void *G, long long V, hipStream_t s) 
 GFIX_INST(double)
 GFIX_INST(float)
 
-void launch_fin_theta(const double *part, long long nb, Ctrl *ctrl, double norm, hipStream_t s) {
-  hipLaunchKernelGGL(k_fin_theta, dim3(1), dim3(1024), 0, s, part, nb, ctrl, norm);
+void launch_fin_theta(const double *part, long long nb, Ctrl *ctrl, double norm, hipStream_t s, int sub) {
+  hipLaunchKernelGGL(k_fin_theta, dim3(1), dim3(1024), 0, s, part, nb, ctrl, norm, sub);
 }
 void launch_fin_pr(const double *part, long long nb, Ctrl *ctrl, hipStream_t s) {
   hipLaunchKernelGGL(k_fin_pr, dim3(1), dim3(1024), 0, s, part, nb, ctrl);
@@ -792,11 +1030,12 @@ void launch_fin_sd(const double *part, long long nb, Ctrl *ctrl, hipStream_t s) 
   hipLaunchKernelGGL(k_fin_sd, dim3(1), dim3(1024), 0, s, part, nb, ctrl);
 }
 void launch_fin_ls(const double *part, long long nb, Ctrl *ctrl, double *trace, int force, double pl1, double pl2,
-                   hipStream_t s) {
-  hipLaunchKernelGGL(k_fin_ls, dim3(1), dim3(1024), 0, s, part, nb, ctrl, trace, force, pl1, pl2);
+                   hipStream_t s, int sub) {
+  hipLaunchKernelGGL(k_fin_ls, dim3(1), dim3(1024), 0, s, part, nb, ctrl, trace, force, pl1, pl2, sub);
 }
-void launch_fin_iter(const double *part, long long nb, Ctrl *ctrl, double *trace, double norm, hipStream_t s) {
-  hipLaunchKernelGGL(k_fin_iter, dim3(1), dim3(1024), 0, s, part, nb, ctrl, trace, norm);
+void launch_fin_iter(const double *part, long long nb, Ctrl *ctrl, double *trace, double norm, hipStream_t s,
+                     int sub) {
+  hipLaunchKernelGGL(k_fin_iter, dim3(1), dim3(1024), 0, s, part, nb, ctrl, trace, norm, sub);
 }
 void launch_sum_part(const double *part, long long nb, double *out, hipStream_t s) {
   hipLaunchKernelGGL(k_sum_part, dim3(1), dim3(1024), 0, s, part, nb, out);
