@@ -136,36 +136,6 @@ template <int WG> __device__ __forceinline__ double bderiv(const double2 *__rest
   return v[0];
 }
 
-// the site's own-link terms of Delta, left by begauge_own in F (the 8
-// accumulators as 4 complex planes), read back by bderiv_rest
-__device__ __forceinline__ void own_store(double2 *__restrict__ F, long long V, long long i, const DerivAcc<double> &d) {
-  F[i] = make_double2(d.R0, d.R1);
-  F[V + i] = make_double2(d.I1, d.R2);
-  F[2 * V + i] = make_double2(d.I2, d.R3);
-  F[3 * V + i] = make_double2(d.R4, d.I4);
-}
-
-// bderiv after begauge_own: the own-link terms from F, the backward
-// neighbours' links added, packed into F in place (each site by its own
-// thread).  The terms are summed in another order than bderiv's.
-template <int WG> __device__ __forceinline__ double bderiv_rest(const double2 *__restrict__ U, double2 *__restrict__ F,
-                                                                const BGeo &g, double (*sh)[kMaxWgWaves]) {
-  double v[1] = {0.0};
-  const long long V = g.V;
-  for (long long i = threadIdx.x; i < V; i += WG) {
-    int x[4];
-    bcoords(g, i, x);
-    DerivAcc<double> d;
-    const double2 p0 = F[i], p1 = F[V + i], p2 = F[2 * V + i], p3 = F[3 * V + i];
-    d.R0 = p0.x, d.R1 = p0.y, d.I1 = p1.x, d.R2 = p1.y, d.I2 = p2.x, d.R3 = p2.y, d.R4 = p3.x, d.I4 = p3.y;
-#pragma unroll 1
-    for (int mu = 0; mu < 4; mu++) d.add_bwd(bload(U, V, bbwd(g, i, x, mu), mu));
-    v[0] += d.store(F, V, i);
-  }
-  wg_sum<WG, 1>(v, sh);
-  return v[0];
-}
-
 // The DFT of N <= 16 numbers in registers (unnormalised; twiddles tw[k] =
 // exp(-2 pi i k / NT) with NT a multiple of N, sign -1 forward): decimation
 // in time by the smallest prime factor R, every index a compile-time
@@ -296,10 +266,10 @@ template <int WG> __device__ __forceinline__ void bdft_axis(double2 *__restrict_
 // in registers, in place.  Every x pencil is
 // padded by one number in LDS (site (x, y, r) at x + (Lx + 1)(y + Ly r)),
 // so that a wave's threads, one pencil each, read and write at a stride
-// that spreads over the LDS banks.  The stage holds 8192 complex numbers
-// (128 KiB) with 512 threads, whose workgroup holds a CU alone, and 4096
+// that spreads over the LDS banks.  The stage holds 9216 complex numbers
+// (144 KiB) with 512 threads, whose workgroup holds a CU alone, and 4608
 // with fewer, whose workgroups share a CU.
-template <int WG> constexpr int stage_cx() { return WG >= 512 ? 8192 : 4096; }
+template <int WG> constexpr int stage_cx() { return WG >= 512 ? 9216 : 4608; }
 
 // whether a slab, padded, fits the stage
 template <int WG> __device__ __forceinline__ bool xyz_staged(const BGeo &g) {
@@ -543,27 +513,71 @@ __device__ __forceinline__ void swap_fields(double2 *&a, double2 *&b) {
   b = t;
 }
 
-// begauge, and the updated links' own-site terms of the next Delta into
-// F (own_store): the next derivative then reads only the backward
-// neighbours' links (bderiv_rest)
+// begauge and bderiv in one pass: U' = g U g^dag in place, the packed Delta
+// of U' into F, the sum of tr Delta^2 returned.  The lattice is walked in
+// chunks of one site per thread, in the order of the sites.  A backward
+// neighbour's U' comes from LDS if the neighbour is in the chunk (along t,
+// where few are, from memory), from memory if its chunk is done, and is
+// otherwise (at the lower edges) formed here from the old link, which nobody
+// replaces before the barrier at the chunk's end.
+// The old links are read once and the new ones written once, where a second
+// pass for the derivative read them again and moved its partial sums twice:
+// 2500 -> 2000 bytes per site and iteration.  Iteration of 512 lattices of
+// 8^4 0.90 -> 0.82 ms, of 96 of 6x10x12x9 0.571 -> 0.560, of 256 of 10^4 1.25
+// -> 1.13, of 64 of 16^4 5.58 -> 5.16.  A barrier per direction, which needs
+// a third of the LDS, drains the loads four times as often: 0.83 and 0.577
+// for the first two.
 template <int WG>
-__device__ __forceinline__ void begauge_own(double2 *__restrict__ U, const double2 *__restrict__ D, double2 *__restrict__ F,
-                                            const BGeo &g, double alpha) {
+__device__ __forceinline__ double begauge_deriv(double2 *__restrict__ U, const double2 *__restrict__ D,
+                                                double2 *__restrict__ F, const BGeo &g, double alpha,
+                                                double (*sh)[kMaxWgWaves], double2 *__restrict__ buf) {
+  static_assert(3 * 6 * WG <= stage_cx<WG>());
+  double v[1] = {0.0};
   const long long V = g.V;
-  for (long long i = threadIdx.x; i < V; i += WG) {
-    int x[4];
-    bcoords(g, i, x);
-    const su3<double> A = bgauge(D, V, i, alpha);
+  const int tid = threadIdx.x;
+  for (long long base = 0; base < V; base += WG) {
+    const long long i = base + tid;
+    const bool on = i < V;
+    int x[4] = {0, 0, 0, 0};
+    su3<double> A;
     DerivAcc<double> d;
+    if (on) {
+      bcoords(g, i, x);
+      A = bgauge(D, V, i, alpha);
 #pragma unroll 1
-    for (int mu = 0; mu < 4; mu++) {
-      const su3<double> m = gtransform<double>(A, bload(U, V, i, mu), bgauge(D, V, bfwd(g, i, x, mu), alpha));
-      bstore(U, V, i, mu, m);
-      d.add_own(m);
+      for (int mu = 0; mu < 4; mu++) {
+        const su3<double> m = gtransform<double>(A, bload(U, V, i, mu), bgauge(D, V, bfwd(g, i, x, mu), alpha));
+        bstore(U, V, i, mu, m);
+        d.add_own(m);
+        if (mu < 3) {
+#pragma unroll
+          for (int k = 0; k < 6; k++) st<double>(buf + (mu * 6 + k) * WG + tid, m.e[kCol01[k]]);
+        }
+      }
     }
-    own_store(F, V, i, d);
+    __syncthreads();
+    if (on) {
+#pragma unroll 1
+      for (int mu = 0; mu < 4; mu++) {
+        const long long xb = bbwd(g, i, x, mu), rel = xb - base;
+        su3<double> m;
+        if (rel >= WG) {
+          m = gtransform<double>(bgauge(D, V, xb, alpha), bload(U, V, xb, mu), A);
+        } else if (rel >= 0 && mu < 3) {
+#pragma unroll
+          for (int k = 0; k < 6; k++) m.e[kCol01[k]] = ld<double>(buf + (mu * 6 + k) * WG + rel);
+          complete_col2(m);
+        } else {
+          m = bload(U, V, xb, mu);
+        }
+        d.add_bwd(m);
+      }
+      v[0] += d.store(F, V, i);
+    }
+    __syncthreads();  // the next chunk's old links and buf may be replaced
   }
-  __syncthreads();
+  wg_sum<WG, 1>(v, sh);
+  return v[0];
 }
 
 struct BTrace {
@@ -646,9 +660,9 @@ __global__ __launch_bounds__(WG, WG >= 256 ? 2 : 1) void k_facg_batch(double2 *c
     long long loc = 0;
     double insum = 0.0, probe[3] = {0.0, 0.0, 0.0};
     int did_ls = 0;
-    int own = 0;  // whether begauge_own left the own-link terms in `in`
+    double next = bderiv<WG>(U, in, g, sh) * norm;
     for (;;) {
-      theta = (own ? bderiv_rest<WG>(U, in, g, sh) : bderiv<WG>(U, in, g, sh)) * norm;
+      theta = next;
       bfourier_accelerate<WG>(in, g, tw, stage);
       bpr_sums<WG>(in, old, g, s2, sh);
       insum = s2[0];
@@ -673,8 +687,7 @@ __global__ __launch_bounds__(WG, WG >= 256 ? 2 : 1) void k_facg_batch(double2 *c
         did_ls = 0;
       }
       swap_fields(in, old);  // in_old <- in
-      begauge_own<WG>(U, sn, in, g, alpha);  // `in` is free until the next derivative
-      own = 1;
+      next = begauge_deriv<WG>(U, sn, in, g, alpha, sh, stage) * norm;  // into `in`, which is free
       tr.rec(theta, alpha, beta);
       loc++;
       if (!(theta > acc && loc < max_iters)) break;
@@ -766,8 +779,9 @@ int facg_batch_run(const size_t dims[4], size_t nlat, double *const *lat, double
   } else if (hipMemcpyAsync(d_lat, lat, nlat * sizeof(double2 *), hipMemcpyHostToDevice, st) != hipSuccess) {
     rc = gfix_fail(-2, "glu_gfix_facg_batch: pointer upload failed");
   } else {
-    // threads per lattice: 512 unless GLU_GFIX_BATCH_WG picks 128 or 256
-    // (512 8^4 lattices: 9350, 8940 and 7080 configs/s at 512, 256 and 128)
+    // threads per lattice: 512 unless GLU_GFIX_BATCH_WG picks 128 or 256,
+    // slower for 512 8^4 lattices (9350, 8940 and 7080 configs/s at 512, 256
+    // and 128 before the update took in the derivative; 22200 at 512 now)
     int wg = 512;
     if (const char *e = getenv("GLU_GFIX_BATCH_WG")) wg = atoi(e);
     auto launch = [&](auto kernel, int threads) {
