@@ -8,9 +8,9 @@
 // stops.
 //
 // On a small lattice the iteration of the context path is bound by the
-// latency of its dozen dependent launches (an 8^4 iteration takes about
-// 75 us of which the bytes account for a few); here one launch carries
-// every iteration of hundreds of lattices.
+// latency of its eight dependent launches (an 8^4 iteration takes 34 us, of
+// which the bytes account for a few); here one launch carries every
+// iteration of hundreds of lattices.
 //
 // Arithmetic is FP64 throughout.  The caller's links (GLU's layout, fixed
 // in place) are copied at the start into device scratch as the first two
@@ -243,22 +243,6 @@ __device__ __forceinline__ void pencil_dft(int N, int sign, const double2 *tw, L
   });
 }
 
-// one DFT along axis mu of every pencil of the 4 fields (sign -1 forward,
-// +1 backward, unnormalised; tw[k] = exp(-2 pi i k / N)) in place in F:
-// the nine-pass form, for slabs beyond the LDS stage
-template <int WG> __device__ __forceinline__ void bdft_axis(double2 *__restrict__ F, const BGeo &g, int mu, int sign, const double2 *tw) {
-  const int N = g.L[mu];
-  const unsigned S = (unsigned)g.S[mu], V = (unsigned)g.V;
-  const unsigned np = V / N;  // pencils per field
-  for (unsigned p = threadIdx.x; p < 4 * np; p += WG) {
-    const unsigned f = p / np, q = p % np;
-    double2 *b = F + (long long)f * V + (q % S) + (q / S) * S * N;
-    pencil_dft(N, sign, tw, [&](int j) { return ld<double>(b + (long long)j * S); },
-               [&](int k, cx<double> v) { st<double>(b + (long long)k * S, v); });
-  }
-  __syncthreads();
-}
-
 // The x, y and z transforms of the time slices of the fields (slabs of
 // Lx Ly Lz sites, contiguous in F) run in LDS, as many slabs at a time as
 // the stage holds: the slabs cross HBM once for the three axes instead of
@@ -268,16 +252,13 @@ template <int WG> __device__ __forceinline__ void bdft_axis(double2 *__restrict_
 // so that a wave's threads, one pencil each, read and write at a stride
 // that spreads over the LDS banks.  The stage holds 9216 complex numbers
 // (144 KiB) with 512 threads, whose workgroup holds a CU alone, and 4608
-// with fewer, whose workgroups share a CU.
+// with fewer, whose workgroups share a CU: a padded slab of 16^3 sites, the
+// largest, fits either.
 template <int WG> constexpr int stage_cx() { return WG >= 512 ? 9216 : 4608; }
+static_assert((kMaxExtent + 1) * kMaxExtent * kMaxExtent <= stage_cx<128>());
 
-// whether a slab, padded, fits the stage
-template <int WG> __device__ __forceinline__ bool xyz_staged(const BGeo &g) {
-  return (long long)(g.L[0] + 1) * g.L[1] * g.L[2] <= stage_cx<WG>();
-}
-
-// x, y, z transforms of the 4 T slabs of the 4 fields (requires
-// xyz_staged); the z sums are written straight back to F
+// x, y, z transforms of the 4 T slabs of the 4 fields; the z sums are
+// written straight back to F
 template <int WG>
 __device__ __forceinline__ void bdft_xyz(double2 *__restrict__ F, const BGeo &g, int sign,
                                          const double2 (*tw)[kMaxExtent], double2 *__restrict__ lds) {
@@ -356,33 +337,10 @@ template <int WG>
 __device__ __forceinline__ void bfourier_accelerate(double2 *__restrict__ F, const BGeo &g,
                                                     const double2 (*tw)[kMaxExtent], double2 *__restrict__ lds) {
   // (one copy of each transform's code for both directions)
-  if (xyz_staged<WG>(g)) {  // three passes over the fields
-#pragma unroll 1
-    for (int sign = -1; sign <= 1; sign += 2) {
-      bdft_xyz<WG>(F, g, sign, tw, lds);
-      if (sign < 0) bdft_t_scale<WG>(F, g, tw);
-    }
-    return;
-  }
 #pragma unroll 1
   for (int sign = -1; sign <= 1; sign += 2) {
-#pragma unroll 1
-    for (int mu = 0; mu < 4; mu++) bdft_axis<WG>(F, g, mu, sign, tw[mu]);
-    if (sign > 0) return;
-    const double mx = 4.0 * 4 / (double)g.V;
-    for (long long i = threadIdx.x; i < g.V; i += WG) {
-      int x[4];
-      bcoords(g, i, x);
-      double kc = 0.0;
-      for (int mu = 0; mu < 4; mu++) kc += tw[mu][x[mu]].x;  // cos(2 pi n / L)
-      const double p2 = (kc == 4.0) ? 1.0 : 2.0 * (4.0 - kc);
-      const double fac = mx / p2;
-      for (int f = 0; f < 4; f++) {
-        const cx<double> z = ld<double>(F + f * g.V + i);
-        st<double>(F + f * g.V + i, mk<double>(z.re * fac, z.im * fac));
-      }
-    }
-    __syncthreads();
+    bdft_xyz<WG>(F, g, sign, tw, lds);
+    if (sign < 0) bdft_t_scale<WG>(F, g, tw);
   }
 }
 
