@@ -737,9 +737,9 @@ int facg_batch_run(const size_t dims[4], size_t nlat, double *const *lat, double
   } else if (hipMemcpyAsync(d_lat, lat, nlat * sizeof(double2 *), hipMemcpyHostToDevice, st) != hipSuccess) {
     rc = gfix_fail(-2, "glu_gfix_facg_batch: pointer upload failed");
   } else {
-    // threads per lattice: 512 unless GLU_GFIX_BATCH_WG picks 128 or 256,
-    // slower for 512 8^4 lattices (9350, 8940 and 7080 configs/s at 512, 256
-    // and 128 before the update took in the derivative; 22200 at 512 now)
+    // threads per lattice: 512 unless GLU_GFIX_BATCH_WG picks 128 or 256
+    // (512 8^4 lattices: 9350, 8940 and 7080 configs/s at 512, 256 and 128
+    // before the update took in the derivative; 10180 at 512 since)
     int wg = 512;
     if (const char *e = getenv("GLU_GFIX_BATCH_WG")) wg = atoi(e);
     auto launch = [&](auto kernel, int threads) {
