@@ -844,12 +844,10 @@ __global__ __launch_bounds__(kBlock) void k_reunit(double2 *__restrict__ U, long
 }
 
 // plaquette / link-trace partial sums: Field/plaqs_links.c:243-265, 399-448.
-// The site's own links are completed once; the twelve neighbour links enter
-// by their two stored columns, and the trace of the two half loops' product
-// by theirs.  Bound by the cache traffic of the neighbour links (1536 B a
-// site, 384 of them from HBM): 385 us on 32^3x64, where full 3x3 products in
-// plain block order took 535; rolled over the six planes at 116 VGPRs it
-// takes 385 too, but 154 against 134 us on 24^3x48.
+// Bound by the cache traffic of the neighbour links (1536 B a site, 384 of
+// them from HBM): 438 us on 32^3x64, 124 on 24^3x48.  Products whose third
+// columns or rows are completed would take 378 and 119, but are off by 1e-7
+// a loop on links rounded to single precision
 __global__ __launch_bounds__(kBlock) void k_measure(const double2 *__restrict__ U, double *__restrict__ part, Geo g) {
   const long long V = g.V;
   const unsigned lb = logical_block(g);
@@ -859,29 +857,24 @@ __global__ __launch_bounds__(kBlock) void k_measure(const double2 *__restrict__ 
   if (i < V) {
     int x[4];
     coords(g, i, x);
-    cx<double> u[4][6], u2[4][3];
+    su3<double> u[4];
 #pragma unroll
     for (int mu = 0; mu < 4; mu++) {
-      load_cols<double>(U, mu, i, V, u[mu]);
-      third_col(u[mu], u2[mu]);
-      const double r = u[mu][0].re + u[mu][4].re + u2[mu][2].re;
+      u[mu] = load_link<double>(U, mu, i, V);
+      const double r = retrace<double>(u[mu]);
       v[1] += r;
       if (mu == 3) v[2] += r;
       mx = r > mx ? r : mx;
     }
+    const long long nb[4] = {nb_fwd(g, i, x, 0), nb_fwd(g, i, x, 1), nb_fwd(g, i, x, 2), nb_fwd(g, i, x, 3)};
 #pragma unroll
     for (int mu = 1; mu < 4; mu++) {
-      const long long t = nb_fwd(g, i, x, mu);
+      const long long t = nb[mu];
 #pragma unroll
-      for (int nu = 0; nu < mu; nu++) {
+      for (int nu = 0; nu < mu; nu++)
         // Re tr(U_mu(x) U_nu(x+mu) U_mu(x+nu)^dag U_nu(x)^dag)
-        cx<double> w[6], P[6], Q[6];
-        load_cols<double>(U, nu, t, V, w);
-        mul_cols01(u[mu], u2[mu], w, P);
-        load_cols<double>(U, mu, nb_fwd(g, i, x, nu), V, w);
-        mul_cols01(u[nu], u2[nu], w, Q);
-        v[0] += retrace_cols(P, Q);
-      }
+        v[0] += retrace_ab_cd_dag<double>(u[mu], load_link<double>(U, nu, t, V), u[nu],
+                                          load_link<double>(U, mu, nb[nu], V));
     }
   }
   __shared__ double mxs[kBlock / kWave];

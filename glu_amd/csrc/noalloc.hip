@@ -71,11 +71,7 @@ __global__ __launch_bounds__(kBlock) void k_na_measure(const double2 *__restrict
       const long long t = nb_fwd(g, i, x, mu);
       for (int nu = 0; nu < mu; nu++) {
         const long long s = nb_fwd(g, i, x, nu);
-        const su3<double> ab = mul_su3<double>(u[mu], load_glu_link(L, t, nu));
-        const su3<double> dc = mul_su3<double>(u[nu], load_glu_link(L, s, mu));
-        double t2 = 0.0;
-        for (int k = 0; k < 9; k++) t2 += ab.e[k].re * dc.e[k].re + ab.e[k].im * dc.e[k].im;
-        v[0] += t2;
+        v[0] += retrace_ab_cd_dag<double>(u[mu], load_glu_link(L, t, nu), u[nu], load_glu_link(L, s, mu));
       }
       d.add(u[mu], load_glu_link(L, nb_bwd(g, i, x, mu), mu));
     }

@@ -204,10 +204,12 @@ __device__ __forceinline__ void mul_cols01(const cx<double> (&A)[6], const cx<do
     for (int r = 0; r < 3; r++)
       m[3 * j + r] = cadd(cadd(cmul(A[r], u[3 * j]), cmul(A[3 + r], u[3 * j + 1])), cmul(a2[r], u[3 * j + 2]));
 }
-// Re tr(M B^dagger) of two SU(3) matrices given by columns 0 and 1: with
-// q_jk = sum_r M_j[r] conj(B_k[r]) the third columns, conj(col0 x col1) of
-// each, enter through the Binet-Cauchy identity as Re(q00 q11 - q01 q10), so
-// neither is formed
+// Re tr(M B^dagger) of two matrices given by columns 0 and 1, the third
+// columns being conj(col0 x col1): with q_jk = sum_r M_j[r] conj(B_k[r])
+// they enter through the Binet-Cauchy identity as Re(q00 q11 - q01 q10), so
+// neither is formed.  For M = A u with u's third column completed that holds
+// only where A is SU(3) to rounding: a reunitarised gauge matrix is, a
+// stored link need not be
 __device__ __forceinline__ double retrace_cols(const cx<double> (&M)[6], const cx<double> (&B)[6]) {
   cx<double> q[2][2];
 #pragma unroll
@@ -320,19 +322,23 @@ template <typename T> __device__ __forceinline__ su3<T> mul_cols(const su3<T> &a
   return o;
 }
 
-// general product a b (rows 0,1; row 2 completed): MMUL/MMUL_SUNC_SSE.c
-template <typename T> __device__ __forceinline__ su3<T> mul_su3(const su3<T> &b, const su3<T> &c) {
-  su3<T> a;
+// Re tr(a b (c d)^dagger), all nine entries of both products formed: links
+// rounded to single precision are SU(3) to 1e-7 only, and a product of which
+// a row or a column is completed from the other two is off by as much
+template <typename T>
+__device__ __forceinline__ T retrace_ab_cd_dag(const su3<T> &a, const su3<T> &b, const su3<T> &c, const su3<T> &d) {
+  T t = T(0);
 #pragma unroll
-  for (int r = 0; r < 2; r++)
+  for (int s = 0; s < 3; s++)
 #pragma unroll
-    for (int s = 0; s < 3; s++)
-      a.e[r * 3 + s] = cadd(cadd(cmul(b.e[r * 3], c.e[s]), cmul(b.e[r * 3 + 1], c.e[3 + s])),
-                            cmul(b.e[r * 3 + 2], c.e[6 + s]));
-  a.e[6] = cconj(csub(cmul(a.e[1], a.e[5]), cmul(a.e[2], a.e[4])));
-  a.e[7] = cconj(csub(cmul(a.e[2], a.e[3]), cmul(a.e[0], a.e[5])));
-  a.e[8] = cconj(csub(cmul(a.e[0], a.e[4]), cmul(a.e[1], a.e[3])));
-  return a;
+    for (int r = 0; r < 3; r++) {
+      const cx<T> p = cadd(cadd(cmul(a.e[r * 3], b.e[s]), cmul(a.e[r * 3 + 1], b.e[3 + s])),
+                           cmul(a.e[r * 3 + 2], b.e[6 + s]));
+      const cx<T> q = cadd(cadd(cmul(c.e[r * 3], d.e[s]), cmul(c.e[r * 3 + 1], d.e[3 + s])),
+                           cmul(c.e[r * 3 + 2], d.e[6 + s]));
+      t += p.re * q.re + p.im * q.im;
+    }
+  return t;
 }
 
 template <typename T> __device__ __forceinline__ T retrace(const su3<T> &m) {
