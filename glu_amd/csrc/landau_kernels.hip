@@ -449,8 +449,8 @@ __device__ __forceinline__ void ls_record(Ctrl *ctrl, const LsStep &r, bool do_l
     for (int k = 0; k < 3; k++) ctrl->probe[k] = r.probe[k];
   ctrl->alpha = r.alpha;
   ctrl->did_ls = do_ls;
+  ctrl->sg_uphill = r.uphill;  // the forced search of an SD start clears it
   if (force) return;
-  ctrl->sg_uphill = r.uphill;
   ctrl->inold = ctrl->insum;  // beta has been taken
 }
 
