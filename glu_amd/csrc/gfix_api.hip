@@ -161,6 +161,7 @@ extern "C" int glu_gfix_create(glu_gfix_ctx **out, const size_t dims[4], int gft
   c->g.Lcu = c->g.S[3];
   geo_set_div(c->g);
   c->g.xcd = 0;
+  if (const char *e = getenv("GLU_GFIX_LS_TILE")) c->ls_rows = atoi(e) < 1 || atoi(e) > 8;  // one tile shape is left
   if (const char *e = getenv("GLU_GFIX_XCD")) {
     c->ord_eg = c->ord_ls = std::min(std::max(atoi(e), 0), 2);
     c->ord_cl = c->ord_eg ? 1 : 0;
@@ -548,9 +549,9 @@ template <typename T> static void enq_update_deriv(glu_gfix_ctx *c, bool fuse) {
 }
 template <typename T> static void enq_line_search(glu_gfix_ctx *c, const void *U, const void *D, int force) {
   if (c->small)
-    launch_line_search_small<T>(U, D, c->part, c->g, c->ctrl, force, c->stream);
+    launch_line_search_small<T>(U, D, c->part, c->g, c->ctrl, force, c->stream, c->ls_rows);
   else
-    launch_line_search<T>(U, D, c->part, geo_order(c, c->ord_ls), c->ctrl, force, c->stream);
+    launch_line_search<T>(U, D, c->part, geo_order(c, c->ord_ls), c->ctrl, force, c->stream, c->ls_rows);
 }
 
 // SD start of steep_Landau_FACG, Gfix/FACG.c:249-265.  sn = in_old = in and

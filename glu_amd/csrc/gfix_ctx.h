@@ -84,6 +84,9 @@ struct glu_gfix_ctx {
   // contiguous and 473 plain, of 24^3x48 134, 138 and 153 us; the line
   // search does not care
   int ord_eg = 2, ord_ls = 1;
+  // FP32 line search with one site per thread in place of its tiles
+  // (launch_line_search); picked by the autotuner, or GLU_GFIX_LS_TILE=0
+  int ls_rows = 0;
   int ord_cl = 1;  // Coulomb slice stencils: XCD-contiguous (1) or plain (0)
   int use_graph = 0;  // replay iteration batches from captured HIP graphs
   // iterations enqueued between host checks; the iterations enqueued past

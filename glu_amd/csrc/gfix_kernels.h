@@ -65,15 +65,18 @@ void launch_cg_update(const void *F, void *sn, long long V, Ctrl *ctrl, hipStrea
                       long long nb = 0);
 template <typename T>
 void launch_copy(const void *F, void *a, long long V, const Ctrl *ctrl, hipStream_t s);
+// whether the FP32 line search has a choice: tiles that divide the lattice,
+// or (rows) one site per thread in the order of the sites
+bool line_search_tiles(const Geo &g);
 template <typename T>
 void launch_line_search(const void *U, const void *F, double *part, const Geo &g, const Ctrl *ctrl, int force,
-                        hipStream_t s);
+                        hipStream_t s, int rows = 0);
 // small lattices: four workgroups of 64 sites in the place of each of 256,
 // whose partial sums stay separate (12 and 4 numbers a row of nblk)
 bool small_lattice(const Geo &g);
 template <typename T>
 void launch_line_search_small(const void *U, const void *F, double *part, const Geo &g, const Ctrl *ctrl, int force,
-                              hipStream_t s);
+                              hipStream_t s, int rows);
 template <typename T>
 void launch_egauge_deriv_small(const void *Uin, void *Uout, const void *D, void *G, void *Fout, double *part,
                                const Geo &g, Ctrl *ctrl, const double *probe, long long nb, hipStream_t s);

@@ -264,8 +264,11 @@ __global__ __launch_bounds__(kBlock) void k_line_search(const vec2<T> *__restric
   block_sum_store<3>(v, part + 3 * lb);
 }
 
-// FP32 links of a shape the tiles do not divide: one probe at a time, the
-// traces from the rows of A u (again for the rounding of the step)
+// FP32 links of a shape the tiles do not divide, or where the autotuner finds
+// this form the faster one: one probe at a time, the traces from the rows of
+// A u (again for the rounding of the step).  On a thermalised 32^3x64 it takes
+// 186 us in contiguous order, the tiles 197; untuned contexts keep the tiles,
+// whose rounding their trajectories follow
 __device__ __forceinline__ su3<double> promote(const su3<float> &m) {
   su3<double> d;
 #pragma unroll
@@ -938,14 +941,13 @@ template <typename T> void launch_copy(const void *F, void *a, long long V, cons
   const unsigned b = (unsigned)std::min<long long>(nblk(n4), 8192);
   hipLaunchKernelGGL(k_copy<T>, dim3(b), dim3(kBlock), 0, s, (const vec2<T> *)F, (vec2<T> *)a, n4, ctrl);
 }
-// whether the FP32 line search's tiles divide the lattice
-static bool probe_tiles(const Geo &g) { return !(g.L[0] % 8 || g.L[1] % 4 || g.L[2] % 4 || g.L[3] % 2); }
+bool line_search_tiles(const Geo &g) { return !(g.L[0] % 8 || g.L[1] % 4 || g.L[2] % 4 || g.L[3] % 2); }
 template <typename T>
 void launch_line_search(const void *U, const void *F, double *part, const Geo &g, const Ctrl *ctrl, int force,
-                        hipStream_t s) {
+                        hipStream_t s, int rows) {
   if constexpr (sizeof(T) == 4) {
     Geo gt = g;
-    if (!probe_tiles(g)) {
+    if (rows || !line_search_tiles(g)) {
       hipLaunchKernelGGL(k_line_search_rows, dim3(nblk(g.V)), dim3(kBlock), 0, s, (const float2 *)U,
                          (const float2 *)F, part, g, ctrl, force);
       return;
@@ -961,10 +963,10 @@ void launch_line_search(const void *U, const void *F, double *part, const Geo &g
 bool small_lattice(const Geo &g) { return nblk(g.V) <= kSmallBlocks; }
 template <typename T>
 void launch_line_search_small(const void *U, const void *F, double *part, const Geo &g, const Ctrl *ctrl, int force,
-                              hipStream_t s) {
+                              hipStream_t s, int rows) {
   const dim3 grid(4 * nblk(g.V)), blk(kBlock);
   if constexpr (sizeof(T) == 4) {
-    if (!probe_tiles(g)) {
+    if (rows || !line_search_tiles(g)) {
       hipLaunchKernelGGL((k_line_search_small<T, PROBE_ROWS>), grid, blk, 0, s, (const vec2<T> *)U,
                          (const vec2<T> *)F, part, g, ctrl, force);
       return;
@@ -1000,12 +1002,12 @@ template <typename T> void launch_identity(void *G, long long V, hipStream_t s) 
   template void launch_cg_update<T>(const void *, void *, long long, Ctrl *, hipStream_t, const double *,      \
                                     long long);                                                               \
   template void launch_line_search_small<T>(const void *, const void *, double *, const Geo &, const Ctrl *,  \
-                                            int, hipStream_t);                                                \
+                                            int, hipStream_t, int);                                           \
   template void launch_egauge_deriv_small<T>(const void *, void *, const void *, void *, void *, double *,    \
                                              const Geo &, Ctrl *, const double *, long long, hipStream_t);    \
   template void launch_copy<T>(const void *, void *, long long, const Ctrl *, hipStream_t);                    \
   template void launch_line_search<T>(const void *, const void *, double *, const Geo &, const Ctrl *, int,   \
-                                      hipStream_t);                                                           \
+                                      hipStream_t, int);                                                      \
   template void launch_egauge<T>(void *, const void *, void *, const Geo &, const Ctrl *, int, hipStream_t);  \
   template void launch_egauge_deriv<T>(const void *, void *, const void *, void *, void *, void *, double *,     \
                                        const Geo &, const Ctrl *, hipStream_t);                                   \

@@ -1,11 +1,13 @@
 // tune.hip -- launch-shape autotuner of a context.
 //
-// The tunable shapes are those that change speed and nothing else:
+// The tunable shapes are those that change speed and, at most, rounding:
 //   - pencils per workgroup of each LDS FFT axis pass (three variants),
 //   - the fused x-y plane pass against two separate axis passes,
 //   - the x values per workgroup of the z-t column pass,
 //   - the workgroup order of the fused update and of the line search
-//     (plain, XCD-contiguous, XCD time slabs).
+//     (plain, XCD-contiguous, XCD time slabs),
+//   - the FP32 line search on tiles against one site per thread (the sums of
+//     the probes then add in another order).
 // glu_gfix_autotune times every candidate with HIP events on the context's
 // own scratch fields (the FFT passes and the derivative write only the
 // field planes and the partial sums) and keeps the fastest.  The choices
@@ -28,7 +30,7 @@ struct Tuning {
   int pv[4];
   int use_xy;
   int zt_pv;
-  int ord_eg, ord_ls;
+  int ord_eg, ord_ls, ls_rows;
   std::string report;
 };
 
@@ -143,24 +145,38 @@ template <typename T> Tuning tune(glu_gfix_ctx *c) {
     void *G = sizeof(T) == 4 ? c->G64 : nullptr;
     const int norder = geo_slab_order_ok(c->g) ? 3 : 2;
     const char *names[3] = {"plain", "XCD-contiguous", "XCD t-slabs"};
-    float eg[3] = {1e30f, 1e30f, 1e30f}, ls[3] = {1e30f, 1e30f, 1e30f};
+    const bool tiles = sizeof(T) == 4 && line_search_tiles(c->g);  // numbered x fastest: no slabs
+    float eg[3] = {1e30f, 1e30f, 1e30f}, ls[3] = {1e30f, 1e30f, 1e30f}, rows[3] = {1e30f, 1e30f, 1e30f};
     for (int o = 0; o < norder; o++) {
       const Geo g = geo_order(c, o);
       eg[o] = time_ms(c, [&] { launch_egauge_deriv<T>(U, Unext, sn, G, Fold, F, c->part, g, dc, c->stream); }, kReps);
-      ls[o] = time_ms(c, [&] { launch_line_search<T>(U, sn, c->part, g, dc, 1, c->stream); }, kReps);
-      snprintf(line, sizeof(line), "order %s: gauge update + derivative %.4f ms, line search %.4f ms\n", names[o],
-               eg[o], ls[o]);
+      snprintf(line, sizeof(line), "order %s: gauge update + derivative %.4f ms", names[o], eg[o]);
       t.report += line;
+      if (!tiles || o < 2) {
+        ls[o] = time_ms(c, [&] { launch_line_search<T>(U, sn, c->part, g, dc, 1, c->stream); }, kReps);
+        snprintf(line, sizeof(line), ", line search %.4f ms%s", ls[o], tiles ? " on tiles" : "");
+        t.report += line;
+      }
+      if (tiles) {
+        rows[o] = time_ms(c, [&] { launch_line_search<T>(U, sn, c->part, g, dc, 1, c->stream, 1); }, kReps);
+        snprintf(line, sizeof(line), ", line search %.4f ms one site per thread", rows[o]);
+        t.report += line;
+      }
+      t.report += "\n";
     }
-    t.ord_eg = t.ord_ls = 0;
-    for (int o = 1; o < norder; o++) {
+    t.ord_eg = t.ord_ls = t.ls_rows = 0;
+    float best_ls = ls[0];
+    for (int o = 0; o < norder; o++) {
       if (eg[o] < eg[t.ord_eg]) t.ord_eg = o;
-      if (ls[o] < ls[t.ord_ls]) t.ord_ls = o;
+      if (ls[o] < best_ls) best_ls = ls[t.ord_ls = o], t.ls_rows = 0;
+      if (rows[o] < best_ls) best_ls = rows[t.ord_ls = o], t.ls_rows = 1;
     }
-    snprintf(line, sizeof(line), "stencil order: update %s, line search %s\n", names[t.ord_eg], names[t.ord_ls]);
+    snprintf(line, sizeof(line), "stencil order: update %s, line search %s%s\n", names[t.ord_eg], names[t.ord_ls],
+             !tiles ? "" : t.ls_rows ? " (one site per thread)" : " (tiles)");
     t.report += line;
   } else {
     t.ord_eg = t.ord_ls = 1;
+    t.ls_rows = c->ls_rows;
   }
   (void)hipStreamSynchronize(c->stream);
   if (dc) (void)hipFree(dc);
@@ -173,6 +189,7 @@ void apply(glu_gfix_ctx *c, const Tuning &t) {
   c->zt_pv = t.zt_pv;
   c->ord_eg = t.ord_eg;
   c->ord_ls = t.ord_ls;
+  c->ls_rows = t.ls_rows;
   for (hipGraphExec_t &gx : c->graph)  // captured launches used the old shapes
     if (gx) {
       (void)hipGraphExecDestroy(gx);
