@@ -7,7 +7,8 @@
 //   - the workgroup order of the fused update and of the line search
 //     (plain, XCD-contiguous, XCD time slabs),
 //   - the FP32 line search on tiles against one site per thread (the sums of
-//     the probes then add in another order).
+//     the probes then add in another order).  Small lattices, whose stencil
+//     kernels take no order, choose this form only.
 // glu_gfix_autotune times every candidate with HIP events on the context's
 // own scratch fields (the FFT passes and the derivative write only the
 // field planes and the partial sums) and keeps the fastest.  The choices
@@ -143,36 +144,52 @@ template <typename T> Tuning tune(glu_gfix_ctx *c) {
     void *sn = sizeof(T) == 4 ? c->sn32 : c->sn;
     void *Fold = sizeof(T) == 4 ? c->old32 : c->old;
     void *G = sizeof(T) == 4 ? c->G64 : nullptr;
-    const int norder = geo_slab_order_ok(c->g) ? 3 : 2;
-    const char *names[3] = {"plain", "XCD-contiguous", "XCD t-slabs"};
     const bool tiles = sizeof(T) == 4 && line_search_tiles(c->g);  // numbered x fastest: no slabs
-    float eg[3] = {1e30f, 1e30f, 1e30f}, ls[3] = {1e30f, 1e30f, 1e30f}, rows[3] = {1e30f, 1e30f, 1e30f};
-    for (int o = 0; o < norder; o++) {
-      const Geo g = geo_order(c, o);
-      eg[o] = time_ms(c, [&] { launch_egauge_deriv<T>(U, Unext, sn, G, Fold, F, c->part, g, dc, c->stream); }, kReps);
-      snprintf(line, sizeof(line), "order %s: gauge update + derivative %.4f ms", names[o], eg[o]);
-      t.report += line;
-      if (!tiles || o < 2) {
-        ls[o] = time_ms(c, [&] { launch_line_search<T>(U, sn, c->part, g, dc, 1, c->stream); }, kReps);
-        snprintf(line, sizeof(line), ", line search %.4f ms%s", ls[o], tiles ? " on tiles" : "");
-        t.report += line;
-      }
+    if (c->small) {
+      // the kernels of small lattices have no order (k_deriv, which only
+      // starts their segments, keeps the context's)
+      t.ord_eg = c->ord_eg;
+      t.ord_ls = c->ord_ls;
       if (tiles) {
-        rows[o] = time_ms(c, [&] { launch_line_search<T>(U, sn, c->part, g, dc, 1, c->stream, 1); }, kReps);
-        snprintf(line, sizeof(line), ", line search %.4f ms one site per thread", rows[o]);
+        float ms[2];
+        for (int r = 0; r < 2; r++)
+          ms[r] = time_ms(c, [&] { launch_line_search_small<T>(U, sn, c->part, c->g, dc, 1, c->stream, r); }, kReps);
+        t.ls_rows = ms[1] < ms[0];
+        snprintf(line, sizeof(line), "small lattice: line search %.4f ms on tiles, %.4f ms in site order\n", ms[0], ms[1]);
         t.report += line;
       }
-      t.report += "\n";
+      snprintf(line, sizeof(line), "stencil order: none on a small lattice%s\n",
+               !tiles ? "" : t.ls_rows ? ", line search in site order" : ", line search on tiles");
+    } else {
+      const int norder = geo_slab_order_ok(c->g) ? 3 : 2;
+      const char *names[3] = {"plain", "XCD-contiguous", "XCD t-slabs"};
+      float eg[3] = {1e30f, 1e30f, 1e30f}, ls[3] = {1e30f, 1e30f, 1e30f}, rows[3] = {1e30f, 1e30f, 1e30f};
+      for (int o = 0; o < norder; o++) {
+        const Geo g = geo_order(c, o);
+        eg[o] = time_ms(c, [&] { launch_egauge_deriv<T>(U, Unext, sn, G, Fold, F, c->part, g, dc, c->stream); }, kReps);
+        snprintf(line, sizeof(line), "order %s: gauge update + derivative %.4f ms", names[o], eg[o]);
+        t.report += line;
+        if (!tiles || o < 2) {
+          ls[o] = time_ms(c, [&] { launch_line_search<T>(U, sn, c->part, g, dc, 1, c->stream); }, kReps);
+          snprintf(line, sizeof(line), ", line search %.4f ms%s", ls[o], tiles ? " on tiles" : "");
+          t.report += line;
+        }
+        if (tiles) {
+          rows[o] = time_ms(c, [&] { launch_line_search<T>(U, sn, c->part, g, dc, 1, c->stream, 1); }, kReps);
+          snprintf(line, sizeof(line), ", line search %.4f ms one site per thread", rows[o]);
+          t.report += line;
+        }
+        t.report += "\n";
+      }
+      float best_ls = ls[0];
+      for (int o = 0; o < norder; o++) {
+        if (eg[o] < eg[t.ord_eg]) t.ord_eg = o;
+        if (ls[o] < best_ls) best_ls = ls[t.ord_ls = o], t.ls_rows = 0;
+        if (rows[o] < best_ls) best_ls = rows[t.ord_ls = o], t.ls_rows = 1;
+      }
+      snprintf(line, sizeof(line), "stencil order: update %s, line search %s%s\n", names[t.ord_eg], names[t.ord_ls],
+               !tiles ? "" : t.ls_rows ? " (one site per thread)" : " (tiles)");
     }
-    t.ord_eg = t.ord_ls = t.ls_rows = 0;
-    float best_ls = ls[0];
-    for (int o = 0; o < norder; o++) {
-      if (eg[o] < eg[t.ord_eg]) t.ord_eg = o;
-      if (ls[o] < best_ls) best_ls = ls[t.ord_ls = o], t.ls_rows = 0;
-      if (rows[o] < best_ls) best_ls = rows[t.ord_ls = o], t.ls_rows = 1;
-    }
-    snprintf(line, sizeof(line), "stencil order: update %s, line search %s%s\n", names[t.ord_eg], names[t.ord_ls],
-             !tiles ? "" : t.ls_rows ? " (one site per thread)" : " (tiles)");
     t.report += line;
   } else {
     t.ord_eg = t.ord_ls = 1;

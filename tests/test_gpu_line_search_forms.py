@@ -47,3 +47,18 @@ def test_autotuner_times_both_forms():
         assert "on tiles" in rep and "one site per thread" in rep, rep
         it, th = g.run(gl.CG, 0.08, 1e-14, 1000)
         assert th < 1e-14 and it < 1000
+
+
+@pytest.mark.parametrize("dims,precision", [((8, 8, 8, 8), gl.FP64), ((8, 8, 8, 8), gl.MIXED), ((6, 6, 6, 10), gl.MIXED)])
+def test_autotuner_times_what_a_small_lattice_runs(dims, precision):
+    """Small lattices (up to 65536 sites) run stencil kernels of their own,
+    without an order of the workgroups: the tuner times none."""
+    print(f"[line search forms] small tuner {dims} {precision}", flush=True)
+    with gl.Gfix(dims, precision=precision) as g:
+        g.heatbath(6.0, 4, 1, seed=3)
+        g.random_transform(seed=4)
+        rep = g.autotune()
+        assert "order plain" not in rep and "stencil order: none" in rep, rep
+        assert ("site order" in rep) == (precision == gl.MIXED and dims[0] % 8 == 0), rep
+        it, th = g.run(gl.CG, 0.08, 1e-14, 1000)
+        assert th < 1e-14 and it < 1000
