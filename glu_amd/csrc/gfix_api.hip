@@ -1146,8 +1146,8 @@ extern "C" int glu_gfix_stage_line_search(glu_gfix_ctx *c, const double *fields,
   if (c->gftype != GLU_GFIX_LANDAU) return gfix_fail(-1, "stage entry points are Landau-only");
   if (int rc = ctrl_live(c, 0.0, 1.0)) return rc;
   if (int rc = fields_in(c, fields, c->sn)) return rc;
-  launch_line_search<double>(c->U64, c->sn, c->part, c->g, c->ctrl, 1, c->stream);
-  launch_fin_ls(c->part, c->nblk, c->ctrl, nullptr, 1, 0.15, 0.30, c->stream);
+  enq_line_search<double>(c, c->U64, c->sn, 1);
+  launch_fin_ls(c->part, c->nblk, c->ctrl, nullptr, 1, 0.15, 0.30, c->stream, part_sub(c));
   if (int rc = read_ctrl(c)) return rc;
   for (int k = 0; k < 3; k++) probes[k] = c->hctrl->probe[k];
   *alpha = c->hctrl->alpha;
