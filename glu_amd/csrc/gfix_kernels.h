@@ -104,7 +104,8 @@ void launch_apply_gauge(void *U, const void *G, const Geo &g, hipStream_t s);
 void launch_promote(const void *a, void *b, long long n, hipStream_t s);
 void launch_reunit(void *U, long long V, int nd, hipStream_t s);
 // the plaquette, link-trace and temporal-trace sums and the largest link
-// trace of the links go to out[0..4)
+// trace of the links go to out[0..4); without out they stay in rows of 4 in
+// part, one for each block of 256 sites
 void launch_measure(const void *U, double *part, double *out, const Geo &g, hipStream_t s);
 
 }  // namespace gfix

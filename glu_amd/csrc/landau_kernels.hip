@@ -1065,7 +1065,8 @@ void launch_reunit(void *U, long long V, int nd, hipStream_t s) {
 }
 void launch_measure(const void *U, double *part, double *out, const Geo &g, hipStream_t s) {
   hipLaunchKernelGGL(k_measure, dim3(nblk(g.V)), dim3(kBlock), 0, s, (const double2 *)U, part, g);
-  hipLaunchKernelGGL(k_fin_measure, dim3(1), dim3(1024), 0, s, part, (long long)nblk(g.V), out);
+  if (out)
+    hipLaunchKernelGGL(k_fin_measure, dim3(1), dim3(1024), 0, s, part, (long long)nblk(g.V), out);
 }
 
 }  // namespace gfix

@@ -2,7 +2,8 @@
 from a single-precision file has them: SU(3) to 1e-7 only, so every product
 has to be formed in full.  Both measurements against the same sums in numpy
 (complex128; the library holds a link's first two columns and completes the
-third), and against each other.
+third), and against each other.  Up to 512 rows of 256 sites the host adds the
+partial sums (16^3x32 is the largest of these), above a second launch does.
 
 Tolerance: 1e-13 relative.  A loop is some tens of roundings of 1.1e-16 and
 sums over thousands of loops average them; a product completed from two of
@@ -44,7 +45,7 @@ def _plaquette(U, dims):
     return 2 * tot / (36 * np.prod(dims))
 
 
-@pytest.mark.parametrize("dims", [(4, 4, 4, 4), (6, 6, 6, 10), (16, 16, 8, 8)])
+@pytest.mark.parametrize("dims", [(4, 4, 4, 4), (6, 6, 6, 10), (16, 16, 8, 8), (16, 16, 16, 32), (12, 10, 42, 40)])
 def test_plaquette_of_single_precision_links(dims):
     print(f"[rounded links] {dims}", flush=True)
     with gl.Gfix(dims, gl.LANDAU, gl.FP64) as g:
