@@ -465,7 +465,10 @@ static bool fast_extent(int N) {
 }
 // axes of 48 and 96 points stay with their compile-time passes in FP32: the
 // three-stage kernels round some products differently, and an FP32
-// trajectory follows the rounding
+// trajectory follows the rounding.  It costs little: an FP32 iteration takes
+// 282, 465, 1058 and 3807 us on 48x12x12x96, 24^3x96, 32^3x96 and 48^3x96,
+// where the run-time passes take 298, 500, 1140 and 4235, and 105 and 76 on
+// 16^3x48 and 10^3x48, where they take 102 and 71
 template <typename T> static bool any_keeps_rounding(const FftAxis &ax) {
   return sizeof(T) == 8 || (ax.N != 48 && ax.N != 96);
 }
@@ -505,6 +508,25 @@ template <typename Need> static int any_split(long long n, int pool, long long l
   return best;
 }
 
+// Two axes that both have compile-time passes: does the run-time pass over
+// both pay?  It saves launches, one of a plane's two or two of a column's
+// three, but its run-time plan costs more per number, so it may pay up to a
+// volume only.  The lines, in sites (4 fields), lie where the times of a
+// whole iteration cross (us with single axes / with the run-time pass):
+//  - x-y planes of up to 64x64 points pay at any volume (32x64x32x32 1128 /
+//    1070 in FP64, 834 / 838 in FP32), larger ones to 2^21 (48x96x16x16 674 /
+//    630, 48x96x24x24 1420 / 1437);
+//  - z-t columns in tiles several sites wide pay at any volume in FP64
+//    (32^2x8x64 253 / 247, 48^2x24^2 688 / 682), to 2^19 in FP32 (230 / 225,
+//    529 / 537);
+//  - columns in tiles one site wide, whose loads are runs of one number, pay
+//    to 2^18 in FP64 (16^3x48 110 / 103, 8^2x64^2 183 / 176, 16^2x32x48 199 /
+//    201, 32^3x96 1575 / 1694, 48^3x96 5.56 / 6.31 ms) and 2^17 in FP32
+//    (8^2x64x32 89 / 88, 16^2x32^2 124 / 124, 48^2x24x64 1325 / 1467).
+static bool any_pays(const FftAxis &a, const FftAxis &b, long long numbers, long long sites) {
+  return !fast_extent(a.N) || !fast_extent(b.N) || numbers <= 4 * sites;
+}
+
 template <typename T, int LAY>
 static void launch_any(void *F, long long fstride, int nfield, const AnyPass &p, unsigned tiles, const PsqInfo &ps,
                        const Ctrl *ctrl, hipStream_t s, int nslice, long long slice_len, const int *slice_done,
@@ -537,6 +559,7 @@ static bool any_plane(void *F, long long fstride, int nfield, const FftAxis &ax,
   auto need = [&](int m) { return 2 * NX * ((m * NY) | 1) + NX + NY; };
   if (!any_keeps_rounding<T>(ax) || !any_keeps_rounding<T>(ay)) return false;
   if ((long long)NX * NY > kAnyPool[2] || need(1) > kAnyPool[2]) return false;
+  if (NX * NY > 4096 && !any_pays(ax, ay, nfield * nslice * nplane * NX * NY, 1 << 21)) return false;
   int m = any_split(nplane, kAnyPool[0], kAnyTiles / ((long long)nfield * nslice) + 1, need);
   if (!m) m = 1;
   AnyPass p{};
@@ -568,9 +591,12 @@ static bool any_column(void *F, long long V, int nfield, const FftAxis &ax, cons
   auto need = [&](int m) { return 2 * NT * ((m * NZ) | 1) + NZ + NT; };
   if (!any_keeps_rounding<T>(az) || !any_keeps_rounding<T>(at)) return false;
   if ((long long)NZ * NT > kAnyPool[2] || need(1) > kAnyPool[2]) return false;
-  if (!launch) return true;
   int m = 0;
   for (int k = 0; k < 3 && !m; k++) m = any_split(nxy, kAnyPool[k], kAnyTiles / nfield, need);
+  if ((sizeof(T) == 4 || m == 1) &&
+      !any_pays(az, at, nfield * V, sizeof(T) == 8 ? 1 << 18 : m == 1 ? 1 << 17 : 1 << 19))
+    return false;
+  if (!launch) return true;
   AnyPass p{};
   p.mode = 2;
   p.m = m;
