@@ -162,6 +162,7 @@ extern "C" int glu_gfix_create(glu_gfix_ctx **out, const size_t dims[4], int gft
   geo_set_div(c->g);
   c->g.xcd = 0;
   if (const char *e = getenv("GLU_GFIX_LS_TILE")) c->ls_rows = atoi(e) < 1 || atoi(e) > 8;  // one tile shape is left
+  if (c->g.L[3] >= 8 * c->g.L[2]) c->ord_eg = 1;
   if (const char *e = getenv("GLU_GFIX_XCD")) {
     c->ord_eg = c->ord_ls = std::min(std::max(atoi(e), 0), 2);
     c->ord_cl = c->ord_eg ? 1 : 0;

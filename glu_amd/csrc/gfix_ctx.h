@@ -82,7 +82,10 @@ struct glu_gfix_ctx {
   // line search; set by the autotuner.  Untuned, the FP64 update of 32^3x64
   // takes 417 us in time slabs (2; 1 where they do not divide), 457
   // contiguous and 473 plain, of 24^3x48 134, 138 and 153 us; the line
-  // search does not care
+  // search does not care.  A slab's blocks find their z neighbours T / 8
+  // slices' blocks away, contiguous ones their t neighbours Lz: where T / 8
+  // is not below Lz a context starts contiguous (FP64 iterations of 16^3x256
+  // 593 us, 614 in slabs, 32^2x8x128 539 and 559; 16^3x128 304 and 302)
   int ord_eg = 2, ord_ls = 1;
   // FP32 line search with one site per thread in place of its tiles
   // (launch_line_search); picked by the autotuner, or GLU_GFIX_LS_TILE=0
