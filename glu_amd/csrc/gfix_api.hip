@@ -118,10 +118,11 @@ void fft_plan(glu_gfix_ctx *c, double2 *const tw[4], double *cosv) {
   c->ps.max = D == 4 ? 4.0 * 4 / (double)V : 4.0 * 3 / (double)c->g.Lcu;
 }
 
-// The transformed axes (x, y, z, and t for Landau) go through the LDS FFT:
-// a workgroup holds P >= 1 pencils of N points (N P <= 2048) and a stage
-// runs at most 1024 butterflies, so N is limited to 2048 and must factor
-// into the radices 2, 3, 5 and 7.
+// The transformed axes (x, y, z, and t for Landau) go through the LDS FFT: a
+// workgroup holds at least one pencil of N points twice, beside its N
+// twiddles, in the largest pool of the run-time pass (10000 numbers), and a
+// plan has at most 8 stages, so N is limited to 2048 and must factor into
+// the radices 2, 3, 5 and 7.
 int check_extents(const size_t dims[4], int gftype) {
   const int D = gftype == GLU_GFIX_LANDAU ? 4 : 3;
   long double vol = 1;

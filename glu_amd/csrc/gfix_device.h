@@ -220,8 +220,9 @@ struct Ctrl {
   long long iters;   // iterations in the current segment
   long long max_iters;
   long long total;   // iterations over all segments (monitoring)
-  // fused gauge updates that ran (counted by the line-search finaliser
-  // that precedes each one); the host compares it with the updates it
+  // fused gauge updates that ran (counted with the step, by the line-search
+  // finaliser that precedes each one or, on small lattices, by the update
+  // itself); the host compares it with the updates it
   // enqueued to put its buffer pointers back after a stop inside a batch
   long long upd;
   int done;          // set after the update of the iteration that stopped
